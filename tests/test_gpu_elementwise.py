@@ -99,3 +99,21 @@ def test_reductions(dev, dt, tol):
     b = K.colsum(d).numpy()
     assert bits_equal(a, b)
     assert rel_err(a, ops.unbroadcast(big, (3072,))) <= tol
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("shape,axes", [((31,), [0]), ((32,), [0]), ((600, 20), [0, 1]), ((8191,), [0]), ((8193,), [0]),
+                                        ((1 << 20,), [0]), ((7, 33), [1]), ((5, 3, 512), [2]), ((5, 3, 513), [1, 2]),
+                                        ((3, 40000), [1]), ((4, 5, 6, 40), [0, 3])])
+def test_sums_over_trailing_axes(dev, dt, shape, axes):
+    """Many terms per output (a loss, a row sum): a group of lanes per output, in
+    parts from 8192 terms on. Bound: n u sum|x| for n added terms, in any order."""
+    D, K = _dev()
+    x = np.random.default_rng(sum(shape)).standard_normal(shape).astype(dt)
+    n = int(np.prod([shape[a] for a in axes]))
+    ref = x.astype(np.longdouble).sum(axis=tuple(axes))
+    bound = n * np.finfo(dt).eps * np.abs(x.astype(np.longdouble)).sum(axis=tuple(axes))
+    assert np.all(np.abs(K.reduce_sum(D.from_numpy(x), axes).numpy() - ref) <= bound)
+    if len(shape) == 2:  # a strided view of the same numbers
+        t = K.reduce_sum(D.from_numpy(np.ascontiguousarray(x.T)).transpose(1, 0), axes).numpy()
+        assert np.all(np.abs(t - ref) <= bound)
