@@ -12,15 +12,17 @@
 // Each operand tile is staged in LDS in its global orientation (global -> LDS
 // is a straight 16-byte vector copy, fully coalesced along the contiguous
 // dimension), with one barrier per k-tile and the next tiles' global loads in
-// flight during the MFMAs. The loads go through per-thread pointers set up
-// once and advanced by one k-tile per load (rows past the matrix edge clamped
-// onto the last row), so the main loop has no index arithmetic and no
-// divergent branches; only a partial last k-tile is masked.
-//   gemm_dma_kernel (16-byte aligned operands -- every GPT-2 GEMM, in float32
-//     and float64): the loads go straight into LDS (global_load_lds_dwordx4)
-//     through three stages, in swizzled layouts that keep the fragment reads
-//     conflict-free.
-//   gemm_kernel (unaligned operands): registers -> LDS, double-buffered.
+// flight during the MFMAs (rows past the matrix edge clamped onto the last row).
+//   gemm_dma_kernel: the loads go straight into LDS (global_load_lds) through
+//     three stages, in swizzled layouts that keep the fragment reads
+//     conflict-free; a wave-uniform base advanced by scalar adds and fixed lane
+//     offsets, so the main loop has no vector instruction but the MFMAs. 16-byte
+//     granular operands (every GPT-2 GEMM, in float32 and float64) take 16 bytes
+//     per lane, others 4: the vocabulary head's products at 50257 columns ran
+//     element by element through registers at 64 to 107 TFLOP/s, and run at 136 to
+//     140 (forward 2961 -> 2256 us, dX 4948 -> 2321, dW 3301 -> 2334).
+//   gemm_kernel (leading dimensions of 2^24 bytes and more): registers -> LDS,
+//     double-buffered.
 //   gemm_x6_kernel (float32 when dtmi_set_gemm_math selects the split-bf16
 //     arithmetic, aligned operands): each operand split exactly into three
 //     bf16 parts on the way into LDS, six partial products on the bf16 MFMA
@@ -45,1087 +47,15 @@
 #include "common.h"
 #include "bufrsrc.h"
 #include "gelu.h"
+#include "gemm_common.h"
 #include "rowln.h"
 
 namespace dtmi {
 
-template <typename T>
-struct MF;
-
-template <>
-struct MF<float> {
-  static constexpr int MT = 32, G = 2, VEC = 4, NACC = 16;
-  typedef float acc_t __attribute__((ext_vector_type(16)));
-  typedef float vec_t __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-  // result register i of lane group g holds row (8*(i/4) + 4*g + i%4), column lane%32
-  static __device__ __forceinline__ int row(int i, int g) { return 8 * (i / 4) + 4 * g + (i % 4); }
-};
-
-template <>
-struct MF<double> {
-  static constexpr int MT = 16, G = 4, VEC = 2, NACC = 4;
-  typedef double acc_t __attribute__((ext_vector_type(4)));
-  typedef double vec_t __attribute__((ext_vector_type(2)));
-  static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  // result register i of lane group g holds row (g + 4*i), column lane%16
-  static __device__ __forceinline__ int row(int i, int g) { return g + 4 * i; }
-};
-
-struct GemmArgs {
-  const void* A;
-  const void* B;
-  void* C;
-  const void* bias;
-  void* ws;  // split-K partials [splits][batch][M][N] (NULL when not split)
-  int64_t M, N, K, lda, ldb, ldc;
-  int64_t sA, sB, sC;  // batch strides (elements)
-  int64_t k_per_split;
-  int tiles_m, tiles_n;
-  int accumulate;
-  // Epilogue fusions (applied after the bias, in this order):
-  const void* addend;  // residual: v = addend[m, n] + v   (row stride ldc)
-  int epi;             // kEpiGeluFwd: aux = gelu(v), C keeps v; kEpiGeluBwd: C = gelu'(aux) * v
-  void* aux;           // [M, N] with row stride ldc
-  // Column sums of B over k (the bias gradient of dW = X^T dY: db = sum over
-  // rows of dY), taken by the blocks of the first row of tiles from the B
-  // tiles already in LDS. Unbatched only. With split-K each split's sums go to
-  // colsum_ws[split][n] and the reduction kernel adds them in split order.
-  void* colsum;
-  void* colsum_ws;
-  int colsum_accumulate;
-};
-
-constexpr int kEpiNone = 0, kEpiGeluFwd = 1, kEpiGeluBwd = 2;
-
-// The fused epilogue of one output element v (the k-sum of row m, column n):
-// bias, residual, accumulate, GELU -- the operation order of the unfused
-// graph (Linear adds its bias, then the residual add, then GELU / its
-// backward as dtrain/autograd.py:133-144 computes them).
-template <typename T>
-__device__ __forceinline__ void epilogue_store(const GemmArgs& a, T* __restrict__ C, int64_t ldc, int64_t m,
-                                               int64_t n, T v, int64_t batch) {
-  if (a.bias) v = v + ((const T*)a.bias)[n];
-  const int64_t o = m * ldc + n;
-  if (a.addend) v = ((const T*)a.addend)[batch * a.sC + o] + v;
-  if (a.accumulate) v = C[o] + v;
-  if (a.epi == kEpiGeluFwd) {
-    ((T*)a.aux)[batch * a.sC + o] = gelu_f<T>(v);
-  } else if (a.epi == kEpiGeluBwd) {
-    v = gelu_b<T>(((const T*)a.aux)[batch * a.sC + o], v);
-  }
-  C[o] = v;
-}
-
-constexpr int kKC = 8;
-// k-tile: 16 floats or 8 doubles
-template <typename T>
-constexpr int kBKT = sizeof(T) == 4 ? 16 : 8;
-
-// One operand tile of BMN rows/columns (along M or N) by kBK.
-template <typename T, bool KCONTIG, int BMN>
-struct TileLayout {
-  static constexpr int VEC = MF<T>::VEC;
-  static constexpr int kBK = kBKT<T>;
-  // k-contiguous: [mn][kBK + VEC]; mn-contiguous: [kBK][BMN + 8]
-  static constexpr int STRIDE = KCONTIG ? (kBK + VEC) : (BMN + 8);
-  static constexpr int SIZE = KCONTIG ? BMN * STRIDE : kBK * STRIDE;
-  static constexpr int NVEC = BMN * kBK / VEC / 256;  // 16-byte vectors per thread per tile
-};
-
-template <typename T, bool KCONTIG, int BMN>
-struct TileRegs {
-  typename MF<T>::vec_t v[TileLayout<T, KCONTIG, BMN>::NVEC];
-};
-
-// Global -> registers for one BMN x kBK operand tile (mn0 = first row/col of
-// the tile along M or N, k0 = first k). Out-of-range elements read as 0.
-template <typename T, bool KCONTIG, int BMN, bool VECLD>
-__device__ __forceinline__ void load_tile(TileRegs<T, KCONTIG, BMN>& r, const T* __restrict__ P, int64_t ld,
-                                          int64_t mn0, int64_t MN, int64_t k0, int64_t kend) {
-  using L = TileLayout<T, KCONTIG, BMN>;
-  constexpr int VEC = L::VEC;
-  constexpr int kBK = L::kBK;
-#pragma unroll
-  for (int i = 0; i < L::NVEC; ++i) {
-    const int f = threadIdx.x + 256 * i;
-    int64_t mn, k;
-    if (KCONTIG) {
-      mn = mn0 + f / (kBK / VEC);
-      k = k0 + (f % (kBK / VEC)) * VEC;
-    } else {
-      k = k0 + f / (BMN / VEC);
-      mn = mn0 + (f % (BMN / VEC)) * VEC;
-    }
-    if (VECLD) {
-      // every dimension that vectors run along is a multiple of VEC
-      if (mn < MN && k < kend) {
-        const T* src = KCONTIG ? P + mn * ld + k : P + k * ld + mn;
-        r.v[i] = *reinterpret_cast<const typename MF<T>::vec_t*>(src);
-      } else {
-        r.v[i] = typename MF<T>::vec_t(0);
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        int64_t mm = KCONTIG ? mn : mn + e;
-        int64_t kk = KCONTIG ? k + e : k;
-        r.v[i][e] = (mm < MN && kk < kend) ? (KCONTIG ? P[mm * ld + kk] : P[kk * ld + mm]) : T(0);
-      }
-    }
-  }
-}
-
-// Per-thread source pointers for the vector loads of the k-tiles that lie
-// wholly inside [kbeg, kend): set up once, advanced by one k-tile per load,
-// so the main loop carries no index arithmetic and no bounds branches. Rows
-// (or columns) past the matrix edge are clamped onto its last row/column:
-// they feed only output rows/columns that the epilogue never stores.
-template <typename T, bool KCONTIG, int BMN>
-struct TilePtr {
-  const T* p[TileLayout<T, KCONTIG, BMN>::NVEC];
-  int64_t step;
-};
-
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void init_ptr(TilePtr<T, KCONTIG, BMN>& t, const T* __restrict__ P, int64_t ld,
-                                         int64_t mn0, int64_t MN, int64_t kbeg) {
-  using L = TileLayout<T, KCONTIG, BMN>;
-  constexpr int VEC = L::VEC;
-  constexpr int kBK = L::kBK;
-#pragma unroll
-  for (int i = 0; i < L::NVEC; ++i) {
-    const int f = threadIdx.x + 256 * i;
-    if (KCONTIG) {
-      int64_t mn = mn0 + f / (kBK / VEC);
-      mn = mn < MN ? mn : MN - 1;
-      t.p[i] = P + mn * ld + kbeg + (f % (kBK / VEC)) * VEC;
-    } else {
-      int64_t mn = mn0 + (f % (BMN / VEC)) * VEC;
-      mn = mn < MN ? mn : MN - VEC;
-      t.p[i] = P + (kbeg + f / (BMN / VEC)) * ld + mn;
-    }
-  }
-  t.step = KCONTIG ? (int64_t)kBK : (int64_t)kBK * ld;
-}
-
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void load_fast(TileRegs<T, KCONTIG, BMN>& r, TilePtr<T, KCONTIG, BMN>& t) {
-#pragma unroll
-  for (int i = 0; i < TileLayout<T, KCONTIG, BMN>::NVEC; ++i) {
-    r.v[i] = *reinterpret_cast<const typename MF<T>::vec_t*>(t.p[i]);
-    t.p[i] += t.step;
-  }
-}
-
-// The last k-tile when it extends past kend: the same number of loads as a
-// full tile, from addresses clamped into [kbeg, kend) (k past kend is zeroed
-// when the tile is stored to LDS, see store_tile_masked).
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void load_tail(TileRegs<T, KCONTIG, BMN>& r, const TilePtr<T, KCONTIG, BMN>& t,
-                                          int64_t ld, int64_t k0, int64_t kend) {
-  using L = TileLayout<T, KCONTIG, BMN>;
-  constexpr int VEC = L::VEC;
-  constexpr int kBK = L::kBK;
-#pragma unroll
-  for (int i = 0; i < L::NVEC; ++i) {
-    const int f = threadIdx.x + 256 * i;
-    const T* q;
-    if (KCONTIG) {
-      const int64_t k = k0 + (f % (kBK / VEC)) * VEC;
-      q = t.p[i] - (k < kend ? 0 : k - (kend - VEC));
-    } else {
-      const int64_t k = k0 + f / (BMN / VEC);
-      q = t.p[i] - (k < kend ? 0 : (k - (kend - 1)) * ld);
-    }
-    r.v[i] = *reinterpret_cast<const typename MF<T>::vec_t*>(q);
-  }
-}
-
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void store_tile(T* __restrict__ lds, const TileRegs<T, KCONTIG, BMN>& r) {
-  using L = TileLayout<T, KCONTIG, BMN>;
-  constexpr int VEC = L::VEC;
-  constexpr int kBK = L::kBK;
-#pragma unroll
-  for (int i = 0; i < L::NVEC; ++i) {
-    const int f = threadIdx.x + 256 * i;
-    int off;
-    if (KCONTIG)
-      off = (f / (kBK / VEC)) * L::STRIDE + (f % (kBK / VEC)) * VEC;
-    else
-      off = (f / (BMN / VEC)) * L::STRIDE + (f % (BMN / VEC)) * VEC;
-    *reinterpret_cast<typename MF<T>::vec_t*>(lds + off) = r.v[i];
-  }
-}
-
-// store_tile for the last, partial k-tile: vectors whose k is at or past
-// kend are stored as zeros.
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void store_tile_masked(T* __restrict__ lds, const TileRegs<T, KCONTIG, BMN>& r,
-                                                  int64_t k0, int64_t kend) {
-  using L = TileLayout<T, KCONTIG, BMN>;
-  constexpr int VEC = L::VEC;
-  constexpr int kBK = L::kBK;
-#pragma unroll
-  for (int i = 0; i < L::NVEC; ++i) {
-    const int f = threadIdx.x + 256 * i;
-    int off;
-    int64_t k;
-    if (KCONTIG) {
-      off = (f / (kBK / VEC)) * L::STRIDE + (f % (kBK / VEC)) * VEC;
-      k = k0 + (f % (kBK / VEC)) * VEC;
-    } else {
-      off = (f / (BMN / VEC)) * L::STRIDE + (f % (BMN / VEC)) * VEC;
-      k = k0 + f / (BMN / VEC);
-    }
-    *reinterpret_cast<typename MF<T>::vec_t*>(lds + off) = k < kend ? r.v[i] : typename MF<T>::vec_t(0);
-  }
-}
-
-// The VEC k-values lane (group g, position c) feeds for operand rows/cols
-// `base + c` at chunk `kk`.
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ typename MF<T>::vec_t read_frag(const T* __restrict__ lds, int base, int kk, int g, int c) {
-  using L = TileLayout<T, KCONTIG, BMN>;
-  constexpr int VEC = L::VEC;
-  typename MF<T>::vec_t v;
-  if (KCONTIG) {
-    v = *reinterpret_cast<const typename MF<T>::vec_t*>(lds + (base + c) * L::STRIDE + kk + VEC * g);
-  } else {
-#pragma unroll
-    for (int s = 0; s < VEC; ++s) v[s] = lds[(kk + VEC * g + s) * L::STRIDE + base + c];
-  }
-  return v;
-}
-
-__device__ __forceinline__ void tile_coords_of(const GemmArgs& a, int t, int& tm, int& tn) {
-  const int nt = a.tiles_m * a.tiles_n;
-  if ((nt & 7) == 0) t = (t & 7) * (nt >> 3) + (t >> 3);  // contiguous tile range per XCD
-  constexpr int GROUP = 8;
-  const int per_group = GROUP * a.tiles_n;
-  const int group = t / per_group;
-  const int first_m = group * GROUP;
-  const int gsz = a.tiles_m - first_m < GROUP ? a.tiles_m - first_m : GROUP;
-  const int r = t - group * per_group;
-  tm = first_m + r % gsz;
-  tn = r / gsz;
-}
-__device__ __forceinline__ void tile_coords(const GemmArgs& a, int& tm, int& tn) {
-  tile_coords_of(a, (int)blockIdx.x, tm, tn);
-}
-
-// The column sum of one B column over this block's k range: to colsum (or
-// added to it), or, with split-K, to the split's row of colsum_ws.
-template <typename T>
-__device__ __forceinline__ void finish_colsum(const GemmArgs& a, double csum, int64_t n, int split) {
-  if (n >= a.N) return;
-  if (a.colsum_ws) {
-    ((T*)a.colsum_ws)[(int64_t)split * a.N + n] = (T)csum;
-  } else {
-    T* cs = (T*)a.colsum;
-    cs[n] = a.colsum_accumulate ? cs[n] + (T)csum : (T)csum;
-  }
-}
-
-// A wave's TM x TN MFMA accumulators (its tile starts at row m0, column n0):
-// split-K partials go to the workspace as they are; otherwise the fused
-// epilogue writes C (and aux).
-template <typename T, int TM, int TN, bool FAST_EPI = false>
-__device__ __forceinline__ void write_acc(const GemmArgs& a, const typename MF<T>::acc_t (&acc)[TM][TN], int64_t m0,
-                                          int64_t n0, int g, int c, int split, int64_t batch) {
-  using MFT = MF<T>;
-  constexpr int MT = MFT::MT, NACC = MFT::NACC;
-  const bool to_ws = a.ws != nullptr;
-  T* C = to_ws ? (T*)a.ws + ((int64_t)split * gridDim.z + batch) * a.M * a.N : (T*)a.C + batch * a.sC;
-  const int64_t ldc = to_ws ? a.N : a.ldc;
-  if constexpr (FAST_EPI && std::is_same<T, float>::value) {
-    if ((to_ws || (a.addend == nullptr && !a.accumulate)) && m0 + TM * MT <= a.M && n0 + TN * MT <= a.N) {
-      // A whole wave tile in range with no residual or accumulation (every
-      // split-K partial, the bias-only products, the GELU epilogues): buffer
-      // accesses off the wave tile's corner -- one lane offset, and per
-      // element a wave-uniform offset, so no per-element address arithmetic
-      // on the SIMD the MFMAs share. The GELU backward's pre-activation of a
-      // row of MFMA tiles is read before its first store (the stores may
-      // alias it as far as the compiler can tell). Same operations as
-      // epilogue_store.
-      const int64_t corner = m0 * ldc + n0;
-      const float* bias = to_ws ? nullptr : (const float*)a.bias;
-      const Rsrc rc = make_rsrc(C + corner, ~0ull);
-      const Rsrc rx = make_rsrc(to_ws ? C : (const float*)a.aux + batch * a.sC + corner, ~0ull);
-      const uint32_t voff = (uint32_t)((4 * g * ldc + c) * 4);
-      auto run = [&](auto modec) {
-        constexpr int MODE = decltype(modec)::value;  // an epilogue kind
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          float x[TN][NACC];
-          if constexpr (MODE == kEpiGeluBwd) {
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-              for (int r = 0; r < NACC; ++r)
-                x[j][r] = buf_load1(rx, voff, (uint32_t)(((i * MT + MFT::row(r, 0)) * ldc + j * MT) * 4));
-          }
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            const float bn = bias ? bias[n0 + j * MT + c] : 0.f;
-#pragma unroll
-            for (int r = 0; r < NACC; ++r) {
-              const uint32_t so = (uint32_t)(((i * MT + MFT::row(r, 0)) * ldc + j * MT) * 4);
-              float v = acc[i][j][r];
-              if (bias) v = v + bn;
-              if constexpr (MODE == kEpiGeluFwd) buf_store1(gelu_f<float>(v), rx, voff, so);
-              if constexpr (MODE == kEpiGeluBwd) v = gelu_b<float>(x[j][r], v);
-              buf_store1(v, rc, voff, so);
-            }
-          }
-        }
-      };
-      const int epi = to_ws ? kEpiNone : a.epi;
-      if (epi == kEpiGeluBwd)
-        run(std::integral_constant<int, kEpiGeluBwd>());
-      else if (epi == kEpiGeluFwd)
-        run(std::integral_constant<int, kEpiGeluFwd>());
-      else
-        run(std::integral_constant<int, kEpiNone>());
-      return;
-    }
-  }
-  const bool plain = to_ws || (a.addend == nullptr && a.epi == kEpiNone && !a.accumulate);
-  if (plain) {  // raw split-K partial, or v + bias
-    const T* bias = to_ws ? nullptr : (const T*)a.bias;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t n = n0 + j * MT + c;
-        if (n >= a.N) continue;
-        const T bn = bias ? bias[n] : T(0);
-#pragma unroll
-        for (int r = 0; r < NACC; ++r) {
-          const int64_t m = m0 + i * MT + MFT::row(r, g);
-          if (m >= a.M) continue;
-          T v = acc[i][j][r];
-          if (bias) v = v + bn;
-          C[m * ldc + n] = v;
-        }
-      }
-  } else {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t n = n0 + j * MT + c;
-        if (n >= a.N) continue;
-#pragma unroll
-        for (int r = 0; r < NACC; ++r) {
-          const int64_t m = m0 + i * MT + MFT::row(r, g);
-          if (m >= a.M) continue;
-          epilogue_store<T>(a, C, ldc, m, n, acc[i][j][r], batch);
-        }
-      }
-  }
-}
-
-// Block tile BM x BN, 4 waves in a 2 x 2 grid of (BM/2) x (BN/2) wave tiles.
-template <typename T, int BM, int BN, bool AKC, bool BKC, bool VECA, bool VECB>
-__global__ void __launch_bounds__(256, 2) gemm_kernel(GemmArgs a) {
-  constexpr int kBK = kBKT<T>;
-  using MFT = MF<T>;
-  using LA = TileLayout<T, AKC, BM>;
-  using LB = TileLayout<T, BKC, BN>;
-  constexpr int MT = MFT::MT, VEC = MFT::VEC, NACC = MFT::NACC;
-  constexpr int WM = BM / 2, WN = BN / 2;
-  constexpr int TM = WM / MT, TN = WN / MT;
-  constexpr int NCH = kBK / kKC;  // 8-wide k chunks per k-tile
-  __shared__ __attribute__((aligned(16))) T lds[2 * (LA::SIZE + LB::SIZE)];
-
-  int tm, tn;
-  tile_coords(a, tm, tn);
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int split = blockIdx.y;
-  const int64_t batch = blockIdx.z;
-  const int64_t kbeg = (int64_t)split * a.k_per_split;
-  const int64_t kend = kbeg + a.k_per_split < a.K ? kbeg + a.k_per_split : a.K;
-  const T* A = (const T*)a.A + batch * a.sA;
-  const T* B = (const T*)a.B + batch * a.sB;
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane / MT, c = lane % MT;
-  const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
-
-  typename MFT::acc_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = typename MFT::acc_t(0);
-
-  // LDS is double-buffered with one barrier per k-tile: iteration kt issues
-  // the global loads of tile kt+1 into registers, computes tile kt from LDS
-  // stage kt&1 while they are in flight, then stores them to the other stage.
-  TileRegs<T, AKC, BM> ra;
-  TileRegs<T, BKC, BN> rb;
-  const int64_t ntiles = kend > kbeg ? (kend - kbeg + kBK - 1) / kBK : 0;
-  const int64_t nfull = kend > kbeg ? (kend - kbeg) / kBK : 0;  // tiles with every k in range
-  TilePtr<T, AKC, BM> pa;
-  TilePtr<T, BKC, BN> pb;
-  if (VECA) init_ptr<T, AKC, BM>(pa, A, a.lda, m0, a.M, kbeg);
-  if (VECB) init_ptr<T, BKC, BN>(pb, B, a.ldb, n0, a.N, kbeg);
-  // Tiles are loaded strictly in order kt = 0, 1, 2, ...; only the last one
-  // can be partial. Every tile issues the same loads with no divergent
-  // branch and no index arithmetic beyond one pointer increment.
-  auto load = [&](int64_t kt, TileRegs<T, AKC, BM>& la, TileRegs<T, BKC, BN>& lb) {
-    const int64_t k0 = kbeg + kt * kBK;
-    if (kt < nfull) {
-      if (VECA) load_fast<T, AKC, BM>(la, pa);
-      if (VECB) load_fast<T, BKC, BN>(lb, pb);
-    } else {
-      if (VECA) load_tail<T, AKC, BM>(la, pa, a.lda, k0, kend);
-      if (VECB) load_tail<T, BKC, BN>(lb, pb, a.ldb, k0, kend);
-    }
-    if (!VECA) load_tile<T, AKC, BM, false>(la, A, a.lda, m0, a.M, k0, kend);
-    if (!VECB) load_tile<T, BKC, BN, false>(lb, B, a.ldb, n0, a.N, k0, kend);
-  };
-  auto store = [&](int64_t kt, int stage, const TileRegs<T, AKC, BM>& sa, const TileRegs<T, BKC, BN>& sb) {
-    T* As = lds + stage * LA::SIZE;
-    T* Bs = lds + 2 * LA::SIZE + stage * LB::SIZE;
-    if (kt < nfull) {
-      store_tile<T, AKC, BM>(As, sa);
-      store_tile<T, BKC, BN>(Bs, sb);
-    } else {
-      const int64_t k0 = kbeg + kt * kBK;
-      store_tile_masked<T, AKC, BM>(As, sa, k0, kend);
-      store_tile_masked<T, BKC, BN>(Bs, sb, k0, kend);
-    }
-  };
-  if (ntiles > 0) {
-    load(0, ra, rb);
-    store(0, 0, ra, rb);
-  }
-  __syncthreads();
-  const bool take_colsum = a.colsum != nullptr && tm == 0 && (int)threadIdx.x < BN;
-  double csum = 0.0;
-  for (int64_t kt = 0; kt < ntiles; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < ntiles) load(kt + 1, ra, rb);
-    const T* As = lds + cur * LA::SIZE;
-    const T* Bs = lds + 2 * LA::SIZE + cur * LB::SIZE;
-#pragma unroll
-    for (int ch = 0; ch < NCH; ++ch) {
-      typename MFT::vec_t fa[TM], fb[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) fa[i] = read_frag<T, AKC, BM>(As, wm0 + i * MT, ch * kKC, g, c);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) fb[j] = read_frag<T, BKC, BN>(Bs, wn0 + j * MT, ch * kKC, g, c);
-#pragma unroll
-      for (int s = 0; s < VEC; ++s)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = MFT::mma(fa[i][s], fb[j][s], acc[i][j]);
-    }
-    if (take_colsum) {
-      // this thread's column of the B tile: its kBK values in k order, then into
-      // the running float64 sum (rows past kend were stored as zeros)
-      T t = T(0);
-#pragma unroll
-      for (int k = 0; k < kBK; ++k) t = t + (BKC ? Bs[threadIdx.x * LB::STRIDE + k] : Bs[k * LB::STRIDE + threadIdx.x]);
-      csum += (double)t;
-    }
-    if (kt + 1 < ntiles) store(kt + 1, cur ^ 1, ra, rb);
-    __syncthreads();
-  }
-  if (take_colsum) finish_colsum<T>(a, csum, n0 + threadIdx.x, split);
-  write_acc<T, TM, TN>(a, acc, m0 + wm0, n0 + wn0, g, c, split, batch);
-}
-
-// ---------------------------------------------------------------------------
-// Direct global -> LDS loads (global_load_lds_dwordx4: each lane fetches 16
-// bytes that land at LDS base + 16 * lane, with no register staging, no LDS
-// store instructions and no wait before a store), float32 and float64 alike:
-// a k-tile is 64 bytes of k per row (16 floats or 8 doubles), VEC = 16 bytes
-// of elements (4 floats or 2 doubles) per vector. Three LDS stages: tile t's
-// loads are issued two iterations before it is computed.
-// LDS layouts (a 1 KB load instruction fills 1 KB contiguously, so conflicts
-// are avoided by choosing which global vector each lane fetches):
-//   KC  (k-contiguous operand, BMN rows x 64 bytes): 1 KB chunks of 16 rows;
-//       the 16-byte k-vector v of chunk row r sits in 16-byte slot
-//       4 r + (v ^ kc_swz(r)), so the 16-byte fragment reads of 16
-//       consecutive rows hit distinct banks;
-//   MNC (mn-contiguous operand, k-rows of BMN elements): k-row k holds its
-//       mn-vectors u at slots u ^ mnc_swz(k), which flips 128 bytes between
-//       the k-rows that the two lane groups of a half-wave fragment read
-//       (k and k + 4 for float32, k and k + 2 for float64), so they hit
-//       different bank halves.
-constexpr int kDmaStages = 3;
-
-__device__ __forceinline__ int kc_swz(int r) { return ((r >> 1) + (r >> 3)) & 3; }
-template <typename T>
-__device__ __forceinline__ int mnc_swz(int k) {
-  return ((k >> (MF<T>::VEC == 4 ? 2 : 1)) & 1) << 3;
-}
-
-// Element offset, within one BMN x 64-byte operand tile, of the 16-byte
-// vector of (row/col mn, k-vector v) for KC, or of (k-row k, mn-vector u)
-// for MNC.
-template <typename T>
-__device__ __forceinline__ int kc_off(int mn, int v) {
-  const int r = mn & 15;
-  return (mn >> 4) * (1024 / (int)sizeof(T)) + (4 * r + (v ^ kc_swz(r))) * MF<T>::VEC;
-}
-template <typename T, int BMN>
-__device__ __forceinline__ int mnc_off(int k, int u) {
-  return k * BMN + (u ^ mnc_swz<T>(k)) * MF<T>::VEC;
-}
-
-// The BMN / 64 load instructions (1 KB each) of each wave per operand tile:
-// a wave-uniform base address (the current k-tile's origin, advanced by
-// scalar adds) and fixed per-lane 32-bit byte offsets, so issuing a tile
-// takes no vector instructions. Offsets are >= 0: clamped rows / columns
-// stay at or after the tile origin (the origin is inside the matrix, and
-// MN - VEC >= mn0 because MN and mn0 are multiples of VEC).
-template <typename T, bool KCONTIG, int BMN>
-struct DmaSrc {
-  static constexpr int NQ = BMN / 64;
-  const T* base;
-  unsigned off[NQ];
-  int64_t step;  // elements per k-tile
-};
-
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void dma_init(DmaSrc<T, KCONTIG, BMN>& s, const T* __restrict__ P, int64_t ld,
-                                         int64_t mn0, int64_t MN, int64_t kbeg, int wave, int lane) {
-  constexpr int NQ = DmaSrc<T, KCONTIG, BMN>::NQ;
-  constexpr int VEC = MF<T>::VEC;
-  constexpr int RV = BMN / VEC;  // mn-vectors per k-row (MNC)
-  s.base = KCONTIG ? P + mn0 * ld + kbeg : P + kbeg * ld + mn0;
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int j = wave * NQ + q;  // 1 KB chunk of the tile
-    if (KCONTIG) {
-      const int r = lane >> 2;
-      int64_t mn = mn0 + 16 * j + r;
-      mn = mn < MN ? mn : MN - 1;
-      const int v = (lane & 3) ^ kc_swz(r);
-      s.off[q] = (unsigned)(((mn - mn0) * ld + VEC * v) * (int64_t)sizeof(T));
-    } else {
-      const int k = (64 * j + lane) / RV;
-      const int u = ((64 * j + lane) % RV) ^ mnc_swz<T>(k);
-      int64_t mn = mn0 + VEC * u;
-      mn = mn < MN ? mn : MN - VEC;
-      s.off[q] = (unsigned)((k * ld + (mn - mn0)) * (int64_t)sizeof(T));
-    }
-  }
-  s.step = KCONTIG ? 64 / (int)sizeof(T) : (64 / (int)sizeof(T)) * ld;
-}
-
-// Issue one operand tile: chunk q of this wave lands at LDS byte address
-// lds_wave + LDS_OFF + 1024 q (lds_wave: wave-uniform, this wave's first
-// chunk of stage 0). m0 takes the LDS address one wait state before the load.
-// The asm writes no SCC (an s_add here would clobber the carry of a 64-bit
-// scalar add the compiler may have split around it): the address is summed
-// outside and moved in with s_mov_b32.
-template <int LDS_OFF, typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void dma_issue(DmaSrc<T, KCONTIG, BMN>& s, unsigned lds_wave) {
-  constexpr int NQ = DmaSrc<T, KCONTIG, BMN>::NQ;
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const unsigned dst = lds_wave + (unsigned)(LDS_OFF + 1024 * q);
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(s.off[q]), "s"(s.base),
-                 "s"(dst)
-                 : "memory", "m0");
-  }
-  s.base += s.step;
-}
-
-// This wave's loads except the newest N have landed, then every wave's have.
-template <int N>
-__device__ __forceinline__ void dma_wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-template <int V>
-struct IC {
-  static constexpr int value = V;
-};
-
-// The partial last k-tile through registers, stored in the same layouts
-// (k at or past kend as zeros).
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void dma_tail_store(T* __restrict__ tile, const TileRegs<T, KCONTIG, BMN>& r, int64_t k0,
-                                               int64_t kend) {
-  using L = TileLayout<T, KCONTIG, BMN>;
-  constexpr int VEC = L::VEC;
-  constexpr int RV = BMN / VEC;
-#pragma unroll
-  for (int i = 0; i < L::NVEC; ++i) {
-    const int f = threadIdx.x + 256 * i;
-    int off;
-    int64_t k;
-    if (KCONTIG) {
-      off = kc_off<T>(f / 4, f % 4);
-      k = k0 + (f % 4) * VEC;
-    } else {
-      off = mnc_off<T, BMN>(f / RV, f % RV);
-      k = k0 + f / RV;
-    }
-    *reinterpret_cast<typename MF<T>::vec_t*>(tile + off) = k < kend ? r.v[i] : typename MF<T>::vec_t(0);
-  }
-}
-
-// Block tile BM x BN (128 or 256 each; 128 x 128 for float64), 4 waves in a
-// 2 x 2 grid of (BM/2) x (BN/2) wave tiles.
-template <typename T, int BM, int BN, bool AKC, bool BKC>
-__global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(GemmArgs a) {
-  using MFT = MF<T>;
-  constexpr int BK = 64 / (int)sizeof(T);
-  constexpr int MT = MFT::MT, VEC = MFT::VEC, LV = VEC == 4 ? 2 : 1;  // VEC = 1 << LV
-  constexpr int WM = BM / 2, WN = BN / 2;
-  constexpr int TM = WM / MT, TN = WN / MT, NCH = BK / kKC;
-  constexpr int TILE_A = BM * BK, TILE_B = BN * BK;  // elements per operand tile
-  constexpr int NST = kDmaStages;
-  __shared__ __attribute__((aligned(1024))) T lds[NST * (TILE_A + TILE_B)];
-
-  int tm, tn;
-  tile_coords(a, tm, tn);
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int split = blockIdx.y;
-  const int64_t batch = blockIdx.z;
-  const int64_t kbeg = (int64_t)split * a.k_per_split;
-  const int64_t kend = kbeg + a.k_per_split < a.K ? kbeg + a.k_per_split : a.K;
-  const T* A = (const T*)a.A + batch * a.sA;
-  const T* B = (const T*)a.B + batch * a.sB;
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane / MT, c = lane % MT;
-  const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
-
-  typename MFT::acc_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = typename MFT::acc_t(0);
-
-  const int ntiles = kend > kbeg ? (int)((kend - kbeg + BK - 1) / BK) : 0;
-  const int nfull = kend > kbeg ? (int)((kend - kbeg) / BK) : 0;
-  DmaSrc<T, AKC, BM> sa;
-  DmaSrc<T, BKC, BN> sb;
-  dma_init<T, AKC, BM>(sa, A, a.lda, m0, a.M, kbeg, wave, lane);
-  dma_init<T, BKC, BN>(sb, B, a.ldb, n0, a.N, kbeg, wave, lane);
-  auto tileA = [&](int st) { return lds + st * (TILE_A + TILE_B); };
-  auto tileB = [&](int st) { return lds + st * (TILE_A + TILE_B) + TILE_A; };
-  // LDS byte address of this wave's first A chunk and first B chunk in stage
-  // 0 (the low 32 bits of a generic LDS address are the LDS offset)
-  const unsigned lds0 = (unsigned)(uintptr_t)lds;
-  const unsigned ldsA = __builtin_amdgcn_readfirstlane(lds0 + wave * DmaSrc<T, AKC, BM>::NQ * 1024u);
-  const unsigned ldsB =
-      __builtin_amdgcn_readfirstlane(lds0 + TILE_A * (unsigned)sizeof(T) + wave * DmaSrc<T, BKC, BN>::NQ * 1024u);
-  constexpr int STAGE_BYTES = (TILE_A + TILE_B) * (int)sizeof(T);
-  constexpr int NQT = DmaSrc<T, AKC, BM>::NQ + DmaSrc<T, BKC, BN>::NQ;  // loads per wave per k-tile
-
-  // Per-lane fragment offsets within a tile: KC fragment (rows base + c,
-  // k-vector (8 / VEC) ch + g); MNC fragment element s (k-row
-  // 8 ch + VEC g + s, column base + c).
-  auto frag = [&](const T* __restrict__ t, bool kcontig, int bmn, int base, int ch) {
-    typename MFT::vec_t v;
-    if (kcontig) {
-      v = *reinterpret_cast<const typename MFT::vec_t*>(t + kc_off<T>(base + c, (kKC / VEC) * ch + g));
-    } else {
-      const int n = base + c;
-#pragma unroll
-      for (int s = 0; s < VEC; ++s) {
-        const int k = kKC * ch + VEC * g + s;
-        v[s] = t[(bmn == 256 ? mnc_off<T, 256>(k, n >> LV) : mnc_off<T, 128>(k, n >> LV)) + (n & (VEC - 1))];
-      }
-    }
-    return v;
-  };
-  const bool take_colsum = a.colsum != nullptr && tm == 0 && (int)threadIdx.x < BN;
-  double csum = 0.0;
-  auto compute = [&](int st) {
-    const T* As = tileA(st);
-    const T* Bs = tileB(st);  // st is a constant in the main loop: immediate LDS offsets
-#pragma unroll
-    for (int ch = 0; ch < NCH; ++ch) {
-      typename MFT::vec_t fa[TM], fb[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) fa[i] = frag(As, AKC, BM, wm0 + i * MT, ch);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) fb[j] = frag(Bs, BKC, BN, wn0 + j * MT, ch);
-#pragma unroll
-      for (int s = 0; s < VEC; ++s)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = MFT::mma(fa[i][s], fb[j][s], acc[i][j]);
-    }
-    if (take_colsum) {
-      // this thread's column of the B tile, its BK values in k order, then
-      // into the running float64 sum (k past kend was stored as zero)
-      const int n = threadIdx.x;
-      T t = T(0);
-#pragma unroll
-      for (int k = 0; k < BK; ++k)
-        t = t + (BKC ? Bs[kc_off<T>(n, k >> LV) + (k & (VEC - 1))] : Bs[mnc_off<T, BN>(k, n >> LV) + (n & (VEC - 1))]);
-      csum += (double)t;
-    }
-  };
-
-  static_assert(NST == 3, "the main loop is unrolled over three stages");
-  auto issue = [&](auto stc) {
-    constexpr int st = decltype(stc)::value;
-    dma_issue<st * STAGE_BYTES>(sa, ldsA);
-    dma_issue<st * STAGE_BYTES>(sb, ldsB);
-  };
-  // One k-tile: this wave's loads of tile kt have landed (the next tile's
-  // may still be in flight), then every wave's have, and every wave is done
-  // with the stage about to be refilled (that of tile kt - 1); then the
-  // loads of tile kt + 2 and the MFMAs of tile kt.
-  auto step = [&](auto stc, int kt) {
-    constexpr int st = decltype(stc)::value;
-    if (kt + 1 < nfull)
-      dma_wait_barrier<NQT>();
-    else
-      dma_wait_barrier<0>();
-    if (kt + 2 < nfull) issue(IC<(st + 2) % 3>());
-    compute(st);
-  };
-  if (nfull > 0) issue(IC<0>());
-  if (nfull > 1) issue(IC<1>());
-  int kt = 0;
-  for (; kt + 3 <= nfull; kt += 3) {
-    step(IC<0>(), kt);
-    step(IC<1>(), kt + 1);
-    step(IC<2>(), kt + 2);
-  }
-  if (kt < nfull) step(IC<0>(), kt);
-  if (kt + 1 < nfull) step(IC<1>(), kt + 1);
-  const int st = nfull % 3;  // stage of the partial tile, if any
-  if (ntiles > nfull) {  // the partial last k-tile, through registers
-    const int64_t k0 = kbeg + (int64_t)nfull * BK;
-    TilePtr<T, AKC, BM> pa;
-    TilePtr<T, BKC, BN> pb;
-    TileRegs<T, AKC, BM> ra;
-    TileRegs<T, BKC, BN> rb;
-    init_ptr<T, AKC, BM>(pa, A, a.lda, m0, a.M, k0);
-    init_ptr<T, BKC, BN>(pb, B, a.ldb, n0, a.N, k0);
-    load_tail<T, AKC, BM>(ra, pa, a.lda, k0, kend);
-    load_tail<T, BKC, BN>(rb, pb, a.ldb, k0, kend);
-    __syncthreads();  // every wave is done with the stage being refilled
-    dma_tail_store<T, AKC, BM>(tileA(st), ra, k0, kend);
-    dma_tail_store<T, BKC, BN>(tileB(st), rb, k0, kend);
-    __syncthreads();
-    compute(st);
-  }
-  if (take_colsum) finish_colsum<T>(a, csum, n0 + threadIdx.x, split);
-  write_acc<T, TM, TN, true>(a, acc, m0 + wm0, n0 + wn0, g, c, split, batch);
-}
-
-// ---------------------------------------------------------------------------
-// float32 products on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16).
-//
-// A float32 x is the exact sum of three bf16 values: x0 = bf16(x), x1 =
-// bf16(x - x0), x2 = x - x0 - x1 (round-to-nearest-even each time; x has 24
-// significant bits and each step takes the leading 8, so x2 is left with at
-// most 8 and bf16 holds it exactly). Then a*b = sum of the 9 products a_i b_j,
-// each exact in float32 (8-bit by 8-bit significands). The kernel adds the 6
-// with i + j <= 2 into float32 MFMA accumulators, smallest first, and drops
-// a1 b2, a2 b1 and a2 b2: |a1| <= 2^-8 |a| and |a2| <= 2^-16 |a|, so what is
-// dropped is below 2^-23 |a b| (about one float32 rounding of the product).
-// The bf16 MFMA runs 16x the float32 MFMA's rate, so the 6 products take
-// 3/8 of the matrix-core time of one float32 MFMA product.
-//
-// Data path: global float32 -> registers (16-byte vectors along k, or 8-byte
-// vectors along m/n for m/n-contiguous operands, 4 k-rows at a time) ->
-// split (v_cvt_pk_bf16_f32, two values per instruction) -> LDS as three bf16
-// planes per operand, each [row][16 k] with the two 16-byte k-halves of a row
-// swapped by a row swizzle, so the MFMA fragment reads (ds_read_b128: lane
-// (g, c) reads row c, k 8g..8g+7) hit distinct banks.
-// k-tile 16 (one MFMA k-step), two LDS stages, one barrier per k-tile.
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-constexpr int kX6BK = 16;
-
-// x and y as three packed bf16 pairs (low half = x): p0 + p1 + p2 == (x, y) exactly.
-// One v_cvt_pk_bf16_f32 per level; the two halves are widened back to float32
-// by bit operations on the packed result (<< 16, & 0xffff0000).
-// (as an asm statement: written as two __bf16 conversions, the compiler
-// rebuilds the low half from a separate one-value conversion)
-__device__ __forceinline__ unsigned cvt_pk_bf16(float x, float y) {
-  unsigned r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
-  return r;
-}
-__device__ __forceinline__ void split3(float x, float y, unsigned& p0, unsigned& p1, unsigned& p2) {
-  p0 = cvt_pk_bf16(x, y);
-  const float rx = x - __uint_as_float(p0 << 16), ry = y - __uint_as_float(p0 & 0xffff0000u);
-  p1 = cvt_pk_bf16(rx, ry);
-  p2 = cvt_pk_bf16(rx - __uint_as_float(p1 << 16), ry - __uint_as_float(p1 & 0xffff0000u));
-}
-
-// The two 16-byte k-halves of a plane row are swapped when bit 2 xor bit 3
-// of the row is set: 8 consecutive rows (and 16) then cover distinct 16-byte
-// bank groups, so 16-byte accesses by consecutive rows are conflict-free
-// whether the LDS serves them 8 or 16 lanes at a time.
-__device__ __forceinline__ int x6_swz(int row) { return ((row >> 2) ^ (row >> 3)) & 1; }
-// byte offset of k-quad kq (k = 4kq..4kq+3) of `row` in one bf16 plane
-__device__ __forceinline__ int x6_quad_off(int row, int kq) {
-  return row * 32 + 16 * ((kq >> 1) ^ x6_swz(row)) + 8 * (kq & 1);
-}
-// byte offset of lane group g's 8 k-values (k = 8g..8g+7) of `row`
-__device__ __forceinline__ int x6_frag_off(int row, int g) { return row * 32 + 16 * (g ^ x6_swz(row)); }
-
-// Splits the 4 consecutive-k values v of `row` (k-quad kq) into the 3 planes.
-template <int PLANE>
-__device__ __forceinline__ void x6_store_quad(char* __restrict__ lds, int row, int kq, float v0, float v1, float v2,
-                                              float v3) {
-  unsigned a0, a1, a2, b0, b1, b2;
-  split3(v0, v1, a0, a1, a2);
-  split3(v2, v3, b0, b1, b2);
-  typedef unsigned u2 __attribute__((ext_vector_type(2)));
-  const int o = x6_quad_off(row, kq);
-  *reinterpret_cast<u2*>(lds + o) = u2{a0, b0};
-  *reinterpret_cast<u2*>(lds + PLANE + o) = u2{a1, b1};
-  *reinterpret_cast<u2*>(lds + 2 * PLANE + o) = u2{a2, b2};
-}
-
-// Splits the 8 consecutive-k values x of `row` (k-half h: k = 8h..8h+7) into
-// the 3 planes: one 16-byte store per plane.
-template <int PLANE>
-__device__ __forceinline__ void x6_store_oct(char* __restrict__ lds, int row, int h, const float (&x)[8]) {
-  typedef unsigned u4 __attribute__((ext_vector_type(4)));
-  u4 p0, p1, p2;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    unsigned a0, a1, a2;
-    split3(x[2 * e], x[2 * e + 1], a0, a1, a2);
-    p0[e] = a0;
-    p1[e] = a1;
-    p2[e] = a2;
-  }
-  const int o = x6_frag_off(row, h);
-  *reinterpret_cast<u4*>(lds + o) = p0;
-  *reinterpret_cast<u4*>(lds + PLANE + o) = p1;
-  *reinterpret_cast<u4*>(lds + 2 * PLANE + o) = p2;
-}
-
-// One operand's BMN x 16 float32 tile. KCONTIG: NV = BMN/64 16-byte vectors
-// per thread (row f/4, k-quad f%4). Otherwise NV = BMN/128 slots per thread of
-// one column (f % BMN) x 8 k-rows (k-half f / BMN), 4-byte loads (a wave
-// reads 64 consecutive columns of a k-row) and one 16-byte LDS store per
-// plane (a wave writes 64 consecutive rows: conflict-free). Addresses are a
-// wave-uniform base (advanced one k-tile per load, in scalar registers) plus
-// per-thread 32-bit byte offsets fixed for the whole k loop; rows or columns
-// past the matrix edge are clamped onto the last ones (they feed only
-// outputs that are never stored). The host keeps every offset below 2^32
-// (leading dimension < 2^22 elements).
-template <bool KCONTIG, int BMN>
-struct X6Src {
-  static constexpr int NV = KCONTIG ? BMN / 64 : BMN / 128;
-  static constexpr int NF = KCONTIG ? 1 : 8;  // loads per vector slot
-  typedef typename std::conditional<KCONTIG, MF<float>::vec_t, float>::type ld_t;
-  const char* base;
-  unsigned off[NV];
-  int64_t ldb;   // bytes between k-rows (n-contiguous operands)
-  int64_t step;  // bytes per k-tile
-  ld_t v[NV][NF];
-
-  __device__ __forceinline__ void init(const float* __restrict__ P, int64_t ld, int64_t mn0, int64_t MN,
-                                       int64_t kbeg) {
-    base = reinterpret_cast<const char*>(KCONTIG ? P + mn0 * ld + kbeg : P + kbeg * ld + mn0);
-    ldb = ld * 4;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int f = threadIdx.x + 256 * i;
-      if constexpr (KCONTIG) {
-        int64_t mn = mn0 + f / 4;
-        mn = mn < MN ? mn : MN - 1;
-        off[i] = (unsigned)(((mn - mn0) * ld + 4 * (f % 4)) * 4);
-      } else {
-        int64_t mn = mn0 + f % BMN;
-        mn = mn < MN ? mn : MN - 1;
-        off[i] = (unsigned)((8 * (f / BMN) * ld + (mn - mn0)) * 4);
-      }
-    }
-    step = (KCONTIG ? (int64_t)kX6BK : (int64_t)kX6BK * ld) * 4;
-  }
-  // a k-tile wholly inside [kbeg, kend)
-  __device__ __forceinline__ void load() {
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-#pragma unroll
-      for (int j = 0; j < NF; ++j) v[i][j] = *reinterpret_cast<const ld_t*>(base + j * ldb + off[i]);
-    base += step;
-  }
-  // the last k-tile, k0 + 16 > kend (k0 = its first k, kend - k0 a multiple
-  // of 4): addresses clamped to the last k-quad (or k-row kend - 1), values
-  // at k >= kend zeroed
-  __device__ __forceinline__ void load_tail(int64_t k0, int64_t kend) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int f = threadIdx.x + 256 * i;
-      if constexpr (KCONTIG) {
-        const int64_t k = k0 + 4 * (f % 4);
-        const int64_t back = k < kend ? 0 : (k - (kend - 4)) * 4;
-        const ld_t x = *reinterpret_cast<const ld_t*>(base + off[i] - back);
-        v[i][0] = k < kend ? x : ld_t(0);
-      } else {
-        const int h = f / BMN;
-        const int64_t col_off = (int64_t)off[i] - 8 * h * ldb;  // the column's byte offset in a k-row
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int64_t k = k0 + 8 * h + j;
-          const int64_t kr = (k < kend ? k : kend - 1) - k0;  // k-row within the tile, clamped
-          const ld_t x = *reinterpret_cast<const ld_t*>(base + kr * ldb + col_off);
-          v[i][j] = k < kend ? x : ld_t(0);
-        }
-      }
-    }
-  }
-  // split the registers into the three planes of the LDS tile
-  __device__ __forceinline__ void store(char* __restrict__ lds) const {
-    constexpr int PLANE = BMN * 32;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int f = threadIdx.x + 256 * i;
-      if constexpr (KCONTIG) {
-        x6_store_quad<PLANE>(lds, f / 4, f % 4, v[i][0][0], v[i][0][1], v[i][0][2], v[i][0][3]);
-      } else {
-        float x[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = v[i][j];
-        x6_store_oct<PLANE>(lds, f % BMN, f / BMN, x);
-      }
-    }
-  }
-  // column sums of an n-contiguous B tile: this thread's column over its 8
-  // k-rows, in k order, into the running float64 sum
-  __device__ __forceinline__ void colsum(double& cs) const {
-    static_assert(!KCONTIG && NV == 1, "column sums: n-contiguous B, 128 columns");
-    float t = v[0][0];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) t = t + v[0][j];
-    cs += (double)t;
-  }
-};
-
-// Block tile BM x BN = 128 x 128, 4 waves in a 2 x 2 grid of 64 x 64 wave tiles.
-template <int BM, int BN, bool AKC, bool BKC>
-__global__ void __launch_bounds__(256, 3) gemm_x6_kernel(GemmArgs a) {
-  static_assert(BM == 128 && BN == 128, "gemm_x6_kernel: 128 x 128 tiles");
-  using MFT = MF<float>;
-  constexpr int MT = 32, WM = BM / 2, WN = BN / 2, TM = WM / MT, TN = WN / MT;
-  constexpr int A_BYTES = 3 * BM * 32, B_BYTES = 3 * BN * 32, STAGE = A_BYTES + B_BYTES;
-  __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
-
-  int tm, tn;
-  tile_coords(a, tm, tn);
-  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-  const int split = blockIdx.y;
-  const int64_t batch = blockIdx.z;
-  const int64_t kbeg = (int64_t)split * a.k_per_split;
-  const int64_t kend = kbeg + a.k_per_split < a.K ? kbeg + a.k_per_split : a.K;
-  const float* A = (const float*)a.A + batch * a.sA;
-  const float* B = (const float*)a.B + batch * a.sB;
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int g = lane / MT, c = lane % MT;
-  const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
-
-  MFT::acc_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = MFT::acc_t(0);
-
-  const int64_t ntiles = kend > kbeg ? (kend - kbeg + kX6BK - 1) / kX6BK : 0;
-  const int64_t nfull = kend > kbeg ? (kend - kbeg) / kX6BK : 0;
-  X6Src<AKC, BM> sa;
-  X6Src<BKC, BN> sb;
-  sa.init(A, a.lda, m0, a.M, kbeg);
-  sb.init(B, a.ldb, n0, a.N, kbeg);
-  bool take_colsum = false;
-  if constexpr (!BKC) take_colsum = a.colsum != nullptr && tm == 0;
-  double cs = 0.0;
-  auto store = [&](int stage) {
-    sa.store(lds + stage * STAGE);
-    sb.store(lds + stage * STAGE + A_BYTES);
-    if constexpr (!BKC)
-      if (take_colsum) sb.colsum(cs);
-  };
-  auto load_tail = [&](int64_t kt) {
-    const int64_t k0 = kbeg + kt * kX6BK;
-    sa.load_tail(k0, kend);
-    sb.load_tail(k0, kend);
-  };
-  auto compute = [&](int stage) {
-    const char* As = lds + stage * STAGE;
-    const char* Bs = As + A_BYTES;
-    bf16x8_t fa[TM][3], fb[TN][3];
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        fa[i][p] = *reinterpret_cast<const bf16x8_t*>(As + p * (BM * 32) + x6_frag_off(wm0 + i * MT + c, g));
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        fb[j][p] = *reinterpret_cast<const bf16x8_t*>(Bs + p * (BN * 32) + x6_frag_off(wn0 + j * MT + c, g));
-    }
-    // partial products smallest first: (2,0) (1,1) (0,2) (1,0) (0,1) (0,0)
-    constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
-#pragma unroll
-    for (int t = 0; t < 6; ++t)
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][PA[t]], fb[j][PB[t]], acc[i][j], 0, 0, 0);
-  };
-  if (ntiles > 0) {
-    if (nfull > 0) {
-      sa.load();
-      sb.load();
-    } else {
-      load_tail(0);
-    }
-    store(0);
-  }
-  __syncthreads();
-  // full k-tiles: the next tile is full too (no bounds work in this loop)
-  int64_t kt = 0;
-  for (; kt + 1 < nfull; ++kt) {
-    sa.load();
-    sb.load();
-    compute((int)(kt & 1));
-    store((int)(kt & 1) ^ 1);
-    __syncthreads();
-  }
-  // the last full tile (its successor, if any, is the partial tail) and the tail
-  for (; kt < ntiles; ++kt) {
-    const bool more = kt + 1 < ntiles;
-    if (more) load_tail(kt + 1);
-    compute((int)(kt & 1));
-    if (more) store((int)(kt & 1) ^ 1);
-    __syncthreads();
-  }
-  if constexpr (!BKC) {
-    if (take_colsum) {
-      // the 2 threads of a column (k-halves 0, 1) add in k order
-      double* red = reinterpret_cast<double*>(lds);
-      red[threadIdx.x] = cs;
-      __syncthreads();
-      if ((int)threadIdx.x < BN) {
-        const int n = threadIdx.x;
-        finish_colsum<float>(a, red[n] + red[BN + n], n0 + n, split);
-      }
-    }
-  }
-  write_acc<float, TM, TN, true>(a, acc, m0 + wm0, n0 + wn0, g, c, split, batch);
-}
+// gemm_f32.hip, gemm_f32_256.hip, gemm_f64.hip, gemm_x6.hip
+template <typename T, int BM, int BN>
+void launch_layout(const GemmArgs& a, dim3 grid, int akc, int bkc, bool veca, bool vecb, bool dma);
+void launch_x6(const GemmArgs& a, dim3 grid, int akc, int bkc);
 
 // Sum of the split-K partials in split order 0, 1, ..., S-1, then the
 // epilogue. PLAIN (bias only): VEC consecutive columns per thread.
@@ -1338,50 +268,9 @@ __global__ void __launch_bounds__(256) splitk_ln_kernel(GemmArgs a, const T* __r
   ln_row_fwd<T, NV, VW>(xv, cols, lane, lw, lb, eps, hout + row * cols, mean + row, rstd + row);
 }
 
-template <typename T, int BM, int BN, bool AKC, bool BKC>
-static void launch_variant(const GemmArgs& a, dim3 grid, bool veca, bool vecb, bool dma) {
-  if (dma) {
-    if constexpr (std::is_same<T, float>::value || (BM == 128 && BN == 128))
-      gemm_dma_kernel<T, BM, BN, AKC, BKC><<<grid, 256, 0, stream()>>>(a);
-    return;
-  }
-  if constexpr (BM != 128 || BN != 128) return;  // larger tiles: aligned float32 only (see gemm_impl)
-  if (veca && vecb)
-    gemm_kernel<T, BM, BN, AKC, BKC, true, true><<<grid, 256, 0, stream()>>>(a);
-  else if (veca)
-    gemm_kernel<T, BM, BN, AKC, BKC, true, false><<<grid, 256, 0, stream()>>>(a);
-  else if (vecb)
-    gemm_kernel<T, BM, BN, AKC, BKC, false, true><<<grid, 256, 0, stream()>>>(a);
-  else
-    gemm_kernel<T, BM, BN, AKC, BKC, false, false><<<grid, 256, 0, stream()>>>(a);
-}
-
-static void launch_x6(const GemmArgs& a, dim3 grid, int akc, int bkc) {
-  if (akc && bkc)
-    gemm_x6_kernel<128, 128, true, true><<<grid, 256, 0, stream()>>>(a);
-  else if (akc)
-    gemm_x6_kernel<128, 128, true, false><<<grid, 256, 0, stream()>>>(a);
-  else if (bkc)
-    gemm_x6_kernel<128, 128, false, true><<<grid, 256, 0, stream()>>>(a);
-  else
-    gemm_x6_kernel<128, 128, false, false><<<grid, 256, 0, stream()>>>(a);
-}
-
 // float32 GEMM arithmetic: DTMI_GEMM_MATH_F32 (float32 MFMA) or
 // DTMI_GEMM_MATH_BF16X6 (exact 3-way bf16 split, 6 bf16 MFMA products).
 static int g_gemm_math = DTMI_GEMM_MATH_F32;
-
-template <typename T, int BM, int BN>
-static void launch_layout(const GemmArgs& a, dim3 grid, int akc, int bkc, bool veca, bool vecb, bool dma) {
-  if (akc && bkc)
-    launch_variant<T, BM, BN, true, true>(a, grid, veca, vecb, dma);
-  else if (akc)
-    launch_variant<T, BM, BN, true, false>(a, grid, veca, vecb, dma);
-  else if (bkc)
-    launch_variant<T, BM, BN, false, true>(a, grid, veca, vecb, dma);
-  else
-    launch_variant<T, BM, BN, false, false>(a, grid, veca, vecb, dma);
-}
 
 struct EpiArgs {
   const void* addend = nullptr;
@@ -1452,6 +341,13 @@ static void pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cu
   }
 }
 
+// k per split: whole k-tiles
+template <typename T>
+static int64_t k_of_splits(int64_t K, int splits) {
+  const int64_t kps = cdiv(cdiv(K, splits), kBKT<T>) * kBKT<T>;
+  return kps < kBKT<T> ? kBKT<T> : kps;
+}
+
 template <typename T>
 static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, int64_t sA,
                      const void* B, int64_t ldb, int64_t sB, void* C, int64_t ldc, int64_t sC, int64_t batch,
@@ -1483,7 +379,7 @@ static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const vo
   // The direct-to-LDS kernel addresses a tile with 32-bit byte offsets from
   // its origin: leading dimensions below 2^24 bytes keep them in range.
   constexpr int64_t kDmaMaxLd = (1 << 24) / (int64_t)sizeof(T);
-  const bool dma = veca && vecb && lda < kDmaMaxLd && ldb < kDmaMaxLd;
+  const bool dma = lda < kDmaMaxLd && ldb < kDmaMaxLd;
   // split-bf16 products: aligned float32 operands (its column sums need an
   // n-contiguous B)
   const bool x6 = std::is_same<T, float>::value && veca && vecb && g_gemm_math == DTMI_GEMM_MATH_BF16X6 &&
@@ -1492,13 +388,11 @@ static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const vo
   if (std::is_same<T, float>::value && dma && !x6) pick_tile(M, N, K, batch, cus, bm, bn);
   const int64_t tmn = cdiv(M, bm) * cdiv(N, bn);
   int splits = force_splits > 0 ? force_splits : choose_splits(tmn, batch, K, cus);
+  const int64_t kps = k_of_splits<T>(K, splits);
   a.tiles_m = (int)cdiv(M, bm);
   a.tiles_n = (int)cdiv(N, bn);
   const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
   DTMI_CHECK(tiles < (1LL << 31) && batch < 65536, "dtmi_gemm: problem too large");
-  constexpr int kBK = kBKT<T>;
-  int64_t kps = cdiv(cdiv(K, splits), kBK) * kBK;
-  if (kps < kBK) kps = kBK;
   splits = (int)cdiv(K > 0 ? K : 1, kps);
   a.k_per_split = kps;
   const size_t es = sizeof(T);
@@ -1539,8 +433,6 @@ static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const vo
         launch_x6(a, grid, akc, bkc);
       else if (bm == 256)
         launch_layout<T, 256, 128>(a, grid, akc, bkc, veca, vecb, dma);
-      else if (bn == 256)
-        launch_layout<T, 128, 256>(a, grid, akc, bkc, veca, vecb, dma);
       else
         launch_layout<T, 128, 128>(a, grid, akc, bkc, veca, vecb, dma);
     } else {
