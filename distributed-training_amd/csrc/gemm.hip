@@ -48,11 +48,12 @@
 #include "bufrsrc.h"
 #include "gelu.h"
 #include "gemm_common.h"
+#include "gemm_direct.h"
 #include "rowln.h"
 
 namespace dtmi {
 
-// gemm_f32.hip, gemm_f32_256.hip, gemm_f64.hip, gemm_x6.hip
+// gemm_f32.hip, gemm_f32_64.hip, gemm_f32_256.hip, gemm_f64.hip, gemm_f64_64.hip, gemm_x6.hip
 template <typename T, int BM, int BN>
 void launch_layout(const GemmArgs& a, dim3 grid, int akc, int bkc, bool veca, bool vecb, bool dma);
 void launch_x6(const GemmArgs& a, dim3 grid, int akc, int bkc);
@@ -341,11 +342,63 @@ static void pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cu
   }
 }
 
+// Estimated time of a plan in SIMD cycles, to compare the 64 x 64 tile and the
+// small-product kernel with the 128-wide tiles. A 32 x 32 piece of the output
+// takes 32 MFMA cycles per k in float32 (32x32x2 in 64 cycles) and 64 in float64
+// (four 16x16x4 of 64 cycles per 4 k); the blocks a CU gets run q = ceil(blocks /
+// CUs) rounds of that. Constants fitted to a sweep of 35 shapes from [64, 768] x
+// [768, 3072] to [2495, 768] x [768, 3072], all layouts, aligned and not, both
+// types (2.2 GHz): a launch costs about 4 us before its first MFMA (3.5 us for the
+// small-product kernel, which waits for no barrier), one block alone on a CU
+// reaches 0.82 (128) or 0.75 (64) of its waves' MFMA rate, several 0.97 to 1 or 0.88,
+// and the small-product kernel 0.45 (float64 0.55): it re-reads its operands for
+// every 32 x 32 tile through the L1. A split adds a launch and its partials'
+// traffic (about 6 TB/s from the last-level cache); where the next pass takes the
+// partials (`fused`: LayerNorm forward or backward, the row dots), only the
+// partials beyond the output itself. Measured, 128 -> chosen:
+// [512, 512] x [512, 128] 23.9 -> 6.0 us (small-product), [1000, 256] x [256, 768]
+// float64 44.6 -> 14 us (small-product), [1500, 384] x [384, 1000] 34 -> 18 us (64),
+// [2495, 768] x [768, 768] 41 -> 29.5 us (64), [1001, 515] x [515, 1030] 36 -> 24 us.
+static double tile_cost(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cus, int bm, int bn, int splits,
+                        size_t es, bool fused) {
+  const double k = (double)cdiv(cdiv(K, splits), 64 / (int64_t)es) * (64.0 / (double)es);
+  const double q = (double)cdiv(cdiv(M, bm) * cdiv(N, bn) * batch * splits, cus);
+  const double eff = bm == 64 ? (q > 1 ? 0.88 : 0.75) : q > 2 ? 0.97 : q > 1 ? 1.0 : 0.82;
+  const double per_k = (es == 4 ? 32.0 : 64.0) * (bm / 32) * (bn / 32) / 4.0;  // four waves
+  double c = 8800.0 + q * k * per_k / eff;
+  const double bytes = (double)(M * N * batch) * (double)es;
+  if (splits > 1) c += fused ? bytes * splits / 2700.0 : 6600.0 + bytes * (splits + 1) / 2700.0;
+  return c;
+}
+
 // k per split: whole k-tiles
 template <typename T>
 static int64_t k_of_splits(int64_t K, int splits) {
   const int64_t kps = cdiv(cdiv(K, splits), kBKT<T>) * kBKT<T>;
   return kps < kBKT<T> ? kBKT<T> : kps;
+}
+
+// GemmArgs::fold_groups of an unsplit or thinly split range: about every 480 k
+// (a group is the 64 x 64 tile's 6 stages)
+template <typename T>
+constexpr int kFoldGroups = sizeof(T) == 4 ? 5 : 10;
+
+// The small-product kernel with kps of k per wave: its loads' rate, or the chain
+// of one wave's MFMAs (which start behind its first loads).
+static double direct_cost(int64_t tiles, int64_t K, int64_t kps, int64_t cus, size_t es) {
+  const double q = (double)cdiv(tiles, cus);
+  const double rate = q * (double)K * (es == 4 ? 8.0 / 0.45 : 16.0 / 0.55);
+  const double chain = 3500.0 + 1.35 * (es == 4 ? 32.0 : 64.0) * (double)kps;
+  return 7700.0 + (rate > chain ? rate : chain);
+}
+
+// k per wave of the small-product kernel when the order of the sum is free:
+// enough waves for 16 per CU, each with at least one batch of k.
+template <typename T>
+static int64_t direct_kps(int64_t tiles, int64_t K, int64_t cus) {
+  int64_t w = 4;
+  while (w < kDirectMaxWaves<T> && tiles * w < 16 * cus) w *= 2;
+  return cdiv(cdiv(K, kDirectBatch<T>), w) * kDirectBatch<T>;
 }
 
 template <typename T>
@@ -388,12 +441,50 @@ static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const vo
   if (std::is_same<T, float>::value && dma && !x6) pick_tile(M, N, K, batch, cus, bm, bn);
   const int64_t tmn = cdiv(M, bm) * cdiv(N, bn);
   int splits = force_splits > 0 ? force_splits : choose_splits(tmn, batch, K, cus);
-  const int64_t kps = k_of_splits<T>(K, splits);
+  bool direct = false;  // the small-product kernel
+  int64_t kps = k_of_splits<T>(K, splits);
+  if (dma && !x6 && force_splits <= 0 && K > 0) {
+    // 7 % below the 128-wide plan's estimate before leaving it
+    const bool fused = ep.ln_out || ep.parts_out || ep.rowdot_out;
+    double best = 0.93 * tile_cost(M, N, K, batch, cus, bm, bn, splits, sizeof(T), fused);
+    const int64_t t32 = cdiv(M, 32) * cdiv(N, 32) * batch;
+    // Float32 products with a dimension of at most 256 (every product of a small
+    // model) keep the 128-wide plan's split of k, and so its bits, whichever kernel
+    // runs: an optimizer's first steps divide gradients by their own size, which
+    // turns another rounding into another trajectory (the second step's gradients
+    // of a 4-layer model of width 128 differed by 3e-6). Others take the fastest.
+    const bool keep = std::is_same<T, float>::value && (M <= 256 || N <= 256 || K <= 256);
+    int64_t dk = kps;
+    if (keep) {
+      const double c = tile_cost(M, N, K, batch, cus, 64, 64, splits, sizeof(T), fused);
+      if (c < best) {
+        best = c;
+        bm = bn = 64;
+      }
+    } else {
+      for (int sp = 1; sp <= 16 && (sp == 1 || K / sp >= 128); ++sp) {
+        const double c = tile_cost(M, N, K, batch, cus, 64, 64, sp, sizeof(T), fused);
+        if (c < best) {
+          best = c;
+          bm = bn = 64;
+          splits = sp;
+          kps = k_of_splits<T>(K, splits);
+          a.fold_groups = kFoldGroups<T>;
+        }
+      }
+      dk = direct_kps<T>(t32, K, cus);
+    }
+    if (cdiv(K, dk) <= kDirectMaxWaves<T> && direct_cost(t32, K, dk, cus, sizeof(T)) < best) {
+      direct = true;
+      splits = 1;
+      kps = dk;
+    }
+  }
   a.tiles_m = (int)cdiv(M, bm);
   a.tiles_n = (int)cdiv(N, bn);
   const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
   DTMI_CHECK(tiles < (1LL << 31) && batch < 65536, "dtmi_gemm: problem too large");
-  splits = (int)cdiv(K > 0 ? K : 1, kps);
+  if (!direct) splits = (int)cdiv(K > 0 ? K : 1, kps);
   a.k_per_split = kps;
   const size_t es = sizeof(T);
   void* ws = nullptr;
@@ -428,7 +519,11 @@ static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const vo
   dim3 grid((unsigned)tiles, (unsigned)splits, (unsigned)batch);
   {
     TimedLaunch tl(DTMI_FAM_GEMM, 2.0 * (double)M * N * K * batch);
-    if constexpr (std::is_same<T, float>::value) {
+    if (direct) {
+      launch_gemm_direct<T>(a, batch, akc, bkc);
+    } else if (bm == 64) {
+      launch_layout<T, 64, 64>(a, grid, akc, bkc, veca, vecb, dma);
+    } else if constexpr (std::is_same<T, float>::value) {
       if (x6)
         launch_x6(a, grid, akc, bkc);
       else if (bm == 256)

@@ -1,4 +1,4 @@
-// Shared by the GEMM kernels: the MFMA shapes, the
+// Shared by the GEMM kernels (gemm.hip, gemm_direct.hip): the MFMA shapes, the
 // launch arguments, the fused epilogue of one element, the block-to-tile order
 // and the column sums' last step.
 #pragma once
@@ -50,6 +50,9 @@ struct GemmArgs {
   int64_t k_per_split;
   int tiles_m, tiles_n;
   int accumulate;
+  // 64 x 64 tile: accumulators added into a second set after every this many
+  // groups of k-tiles (0: one chain over the whole k range)
+  int fold_groups;
   // Epilogue fusions (applied after the bias, in this order):
   const void* addend;  // residual: v = addend[m, n] + v   (row stride ldc)
   int epi;             // kEpiGeluFwd: aux = gelu(v), C keeps v; kEpiGeluBwd: C = gelu'(aux) * v

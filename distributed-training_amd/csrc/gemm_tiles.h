@@ -348,8 +348,10 @@ __global__ void __launch_bounds__(256, 2) gemm_kernel(GemmArgs a) {
 //       the k-rows that the two lane groups of a half-wave fragment read
 //       (k and k + 4 for float32, k and k + 2 for float64), so they hit
 //       different bank halves.
+// The 64 x 64 tile has a quarter of the MFMAs to cover a load with, so it keeps
+// more tiles in flight.
 template <int BM, int BN>
-constexpr int kDmaStages = 3;
+constexpr int kDmaStages = BM == 64 && BN == 64 ? 6 : 3;
 
 __device__ __forceinline__ int kc_swz(int r) { return ((r >> 1) + (r >> 3)) & 3; }
 template <typename T>
@@ -496,7 +498,7 @@ __device__ __forceinline__ void dma_tail_store(T* __restrict__ tile, const TileR
   }
 }
 
-// Block tile BM x BN (128 x 128, or 256 x 128 in float32), 4 waves in a
+// Block tile BM x BN (64 x 64, 128 x 128, or 256 x 128 in float32), 4 waves in a
 // 2 x 2 grid of (BM/2) x (BN/2) wave tiles.
 template <typename T, int BM, int BN, bool AKC, bool BKC, bool VECA, bool VECB>
 __global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(GemmArgs a) {
@@ -630,8 +632,35 @@ __global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(
     constexpr int st = decltype(stc)::value;
     if (st < NST - 1 && st < nfull) issue(stc);
   });
-  int kt = 0;
-  for (; kt + NST <= nfull; kt += NST) each_stage([&](auto stc) { step(stc, kt + decltype(stc)::value); });
+  // A long range without a K split is summed in pieces (a.fold_groups): a chain
+  // of thousands of float32 additions would lose what the splits of the 128-wide
+  // tiles keep. 32 vector instructions per 480 k, 1 % of the MFMA time.
+  constexpr bool FOLD = BM == 64;
+  typename MFT::acc_t tot[FOLD ? TM : 1][FOLD ? TN : 1];
+  if constexpr (FOLD)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) tot[i][j] = typename MFT::acc_t(0);
+  auto fold = [&]() {
+    if constexpr (FOLD)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          tot[i][j] += acc[i][j];
+          acc[i][j] = typename MFT::acc_t(0);
+        }
+  };
+  int kt = 0, grp = 0;
+  for (; kt + NST <= nfull; kt += NST) {
+    each_stage([&](auto stc) { step(stc, kt + decltype(stc)::value); });
+    if constexpr (FOLD)
+      if (++grp == a.fold_groups) {
+        fold();
+        grp = 0;
+      }
+  }
   each_stage([&](auto stc) {
     if (kt + decltype(stc)::value < nfull) step(stc, kt + decltype(stc)::value);
   });
@@ -660,6 +689,12 @@ __global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(
     __syncthreads();
     compute(st);
   }
+  if constexpr (FOLD)
+    if (a.fold_groups > 0)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += tot[i][j];
   if (take_colsum) finish_colsum<T>(a, csum, n0 + threadIdx.x, split);
   write_acc<T, TM, TN, true>(a, acc, m0 + wm0, n0 + wn0, g, c, split, batch);
 }

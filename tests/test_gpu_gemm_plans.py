@@ -1,0 +1,74 @@
+"""The GEMM kernels behind the dispatch's size rules: the small-product kernel (k
+split over a block's waves), the 64 x 64 tile and the 4-byte loads of operands
+that are not 16-byte granular, at tile edges, remainders and both ends of their
+ranges, in every layout. The reference is a float64 product. The bounds are the
+worst case of a sum of K products, K u |A||B| (u the unit roundoff, eps = 2 u:
+the other half covers the float64 reference's own sum), which a lost or doubled
+term exceeds by orders of magnitude."""
+import numpy as np
+import pytest
+
+from helpers import bits_equal
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [(True, False), (True, True), (False, False), (False, True)]
+
+
+def _operands(dt, M, N, K, akc, bkc, seed):
+    rng = np.random.default_rng(seed)
+    A = rng.standard_normal((M, K) if akc else (K, M)).astype(dt)
+    B = rng.standard_normal((N, K) if bkc else (K, N)).astype(dt)
+    a = (A if akc else A.T).astype(np.float64)
+    b = (B.T if bkc else B).astype(a.dtype)
+    return A, B, a, b
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 1), (33, 31, 7), (32, 64, 32), (512, 128, 128), (128, 384, 511), (201, 65, 385),  # small products
+    (257, 259, 261), (320, 512, 300), (300, 700, 2050),  # 64 x 64 tiles, with and without splits and folds
+    (1031, 1029, 515),  # odd in every dimension
+])
+def test_gemm_plans_against_reference(dev, dt, akc, bkc, M, N, K):
+    from dtmi import device as D, kernels as K_
+    A, B, a, b = _operands(dt, M, N, K, akc, bkc, M * 7 + N * 3 + K)
+    bias = np.random.default_rng(1).standard_normal(N).astype(dt)
+    got = K_.gemm(D.from_numpy(A), D.from_numpy(B), a_kcontig=akc, b_kcontig=bkc, bias=D.from_numpy(bias)).numpy()
+    bound = np.finfo(dt).eps * (K * (np.abs(a) @ np.abs(b)) + np.abs(bias))
+    assert np.all(np.abs(got - (a @ b + bias)) <= bound)
+
+
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+@pytest.mark.parametrize("M,N,K,splits", [(512, 128, 128, 1), (512, 128, 512, 2), (96, 65, 200, 1), (65, 2000, 777, 3),
+                                          (1000, 130, 1920, 7), (250, 1030, 515, 2)])
+def test_small_float32_products_keep_the_wide_tiles_bits(dev, akc, bkc, M, N, K, splits):
+    """A float32 product with a dimension of at most 256 gives the bits of the
+    128-wide tiles at their own split of k, whichever kernel takes it."""
+    from dtmi import device as D, kernels as K_
+    A, B, _, _ = _operands(np.float32, M, N, K, akc, bkc, K)
+    da, db = D.from_numpy(A), D.from_numpy(B)
+    got = K_.gemm(da, db, a_kcontig=akc, b_kcontig=bkc).numpy()
+    assert bits_equal(got, K_.gemm(da, db, a_kcontig=akc, b_kcontig=bkc, splits=splits).numpy())
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("M,K,N", [(512, 128, 384), (77, 33, 65), (1000, 256, 768), (2495, 300, 513)])
+def test_linear_backward_column_sums_and_epilogues(dev, dt, M, K, N):
+    """dW, db and dX, and the fused forward epilogues, through the small plans."""
+    from dtmi import device as D, kernels as K_
+    rng = np.random.default_rng(M + N)
+    x, w, g = (rng.standard_normal(s).astype(dt) for s in ((M, K), (K, N), (M, N)))
+    b, r = rng.standard_normal(N).astype(dt), rng.standard_normal((M, N)).astype(dt)
+    X, W, G = (v.astype(np.float64) for v in (x, w, g))
+    eps = np.finfo(dt).eps
+    dx, dw, db = K_.linear_bwd(D.from_numpy(x), D.from_numpy(w), D.from_numpy(g))
+    assert np.all(np.abs(dx.numpy() - G @ W.T) <= eps * N * (np.abs(G) @ np.abs(W.T)))
+    assert np.all(np.abs(dw.numpy() - X.T @ G) <= eps * M * (np.abs(X.T) @ np.abs(G)))
+    assert np.all(np.abs(db.numpy() - G.sum(0)) <= eps * M * np.abs(G).sum(0))
+    y, _ = K_.linear_fwd_fused(D.from_numpy(x), D.from_numpy(w), D.from_numpy(b), residual=D.from_numpy(r))
+    bound = eps * (K * (np.abs(X) @ np.abs(W)) + np.abs(b) + 2 * np.abs(r))
+    assert np.all(np.abs(y.numpy() - (X @ W + b + r)) <= bound)
+    h, act = K_.linear_fwd_fused(D.from_numpy(x), D.from_numpy(w), D.from_numpy(b), gelu=True)
+    assert bits_equal(act.numpy(), K_.gelu_fwd(h).numpy())
