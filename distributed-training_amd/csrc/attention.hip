@@ -25,7 +25,7 @@
 // registers) and writing dS = P * (dP - rowsum(dO * O)) to a [B, H, T, T]
 // workspace; kernel B owns queries and accumulates dQ = dS K from it (when
 // the workspace would exceed its bound, kernel B recomputes dS instead).
-// Float32 with D = 64 and T a multiple of 32 works on 16 x 16 tiles with
+// Float32 with D of 36 to 128 works on 16 x 16 tiles with
 // paired ranges: key tile j and its mirror nt - 1 - j (nt + 1 tile pairs
 // between them) split over two waves in the key pass, query tile i and its
 // mirror over a pair of waves in the dQ pass, so every wave carries the same
@@ -1073,7 +1073,8 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_kernel(AttnArgs a) {
 }
 
 // ------------------------------------------- head dimensions beyond 64
-// For D > 64 the scores of one batch element are materialised, [H, T, T] in
+// Where no other form applies (float64, float32 above D = 128, unaligned rows
+// or a dS above its bound) the scores of one batch element are materialised, [H, T, T] in
 // a pooled workspace, and the products run as batched GEMMs (dtmi_gemm):
 // S = Q K^T, P = softmax(S * scale + mask), O = P V; backward P recomputed
 // from S and the saved row statistics, dV = P^T dO, dP = dO V^T,
@@ -1102,68 +1103,98 @@ __device__ __forceinline__ VT buf_load_v(Rsrc r, uint32_t voff, uint32_t soff) {
   static_assert(sizeof(VT) == 16, "16-byte vectors");
   return __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
 }
-// dK (times the softmax scale) and dV of 16 keys from the key pass's
-// accumulators: lane (g, c), tile t, register i holds key k0 + c,
-// d = 4 row(i, g) + t.
-template <typename T>
-__device__ __forceinline__ void store_kv16(const AttnArgs& a, int64_t b, int64_t h, int k0,
-                                           const typename A16<T>::acc_t (&dk)[4],
-                                           const typename A16<T>::acc_t (&dv)[4], int g, int c) {
-  using M = A16<T>;
-  T* DK = (T*)a.dk + b * a.sdk.b + h * a.sdk.h + (int64_t)(k0 + c) * a.sdk.t;
-  T* DV = (T*)a.dv + b * a.sdv.b + h * a.sdv.h + (int64_t)(k0 + c) * a.sdv.t;
-  const T scale = (T)a.scale;
+
+// Geometry of the paired-range kernels for head dimensions up to DP (64, 96
+// or 128): N d-tiles of 16; a lane's slice of a row is SL = DP / 4 elements; a
+// wave's 16-byte loads of a 16-row tile take CPV columns by RPV rows each, NCB
+// column groups (DP = 64: whole rows; 96 and 128: 32 columns, 8 rows).
+template <int DP>
+struct P16 {
+  static_assert(DP == 64 || DP == 96 || DP == 128, "padded head dimensions");
+  static constexpr int N = DP / 16, SL = DP / 4, NF = SL / 4;
+  static constexpr int LD = DP + 4, TILE = 16 * LD;
+  static constexpr int CPV = DP == 64 ? 64 : 32, NCB = DP / CPV, RPV = 256 / CPV, NV = 16 * DP / 256;
+};
+// Byte offset past every buffer's end (extents stay below 2^31 on the ragged
+// path, and so do the offsets added to it): loads there return zero.
+constexpr uint32_t kOutside = 0x80000000u;
+
+// RAG: T any length, D any multiple of 4 up to DP. Rows past T and columns
+// past D read as zero through the buffer's bounds, which hold for the vector
+// offset, so a tile's offset goes there and not into the scalar one.
+template <bool RAG, typename VT>
+__device__ __forceinline__ VT load_at(Rsrc r, uint32_t voff, uint32_t tile) {
+  if constexpr (RAG) return buf_load_v<VT>(r, voff + tile, 0);
+  return buf_load_v<VT>(r, voff, tile);
+}
+template <bool RAG>
+__device__ __forceinline__ Rsrc rows_rsrc(const float* base, int64_t Tn, int64_t rs, int64_t D) {
+  return make_rsrc(base, (uint64_t)(RAG ? (Tn - 1) * rs + D : Tn * rs) * 4);
+}
+// N consecutive floats of LDS (16-byte aligned for N a multiple of 4, else 8-byte)
+template <int N>
+__device__ __forceinline__ void lds_row(float (&x)[N], const float* p) {
+  constexpr int W = N % 4 == 0 ? 4 : 2;
+  typedef float vt __attribute__((ext_vector_type(W)));
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = 4 * M::row(i, g);
-    const typename M::acc_t xk = {dk[0][i] * scale, dk[1][i] * scale, dk[2][i] * scale, dk[3][i] * scale};
-    const typename M::acc_t xv = {dv[0][i], dv[1][i], dv[2][i], dv[3][i]};
-    if (a.ovec) {
+  for (int v = 0; v < N / W; ++v) {
+    const vt y = *reinterpret_cast<const vt*>(p + W * v);
 #pragma unroll
-      for (int v = 0; v < 4 / M::VEC; ++v) {
-        typename M::vec_t yk, yv;
+    for (int e = 0; e < W; ++e) x[W * v + e] = y[e];
+  }
+}
+// N consecutive results at column d of a row, those below D; vec: the row is
+// 16-byte aligned (d is a multiple of N)
+template <int N, bool RAG>
+__device__ __forceinline__ void put_row(float* row, int d, int D, const float (&x)[N], bool vec) {
+  constexpr int W = N % 4 == 0 ? 4 : 2;
+  typedef float vt __attribute__((ext_vector_type(W)));
 #pragma unroll
-        for (int e = 0; e < M::VEC; ++e) {
-          yk[e] = xk[M::VEC * v + e];
-          yv[e] = xv[M::VEC * v + e];
-        }
-        *reinterpret_cast<typename M::vec_t*>(DK + d + M::VEC * v) = yk;
-        *reinterpret_cast<typename M::vec_t*>(DV + d + M::VEC * v) = yv;
-      }
+  for (int v = 0; v < N / W; ++v) {
+    const int dv = d + W * v;
+    if (RAG && dv >= D) continue;  // D is a multiple of 4 here, so vectors are wholly in or out
+    if (vec) {
+      vt y;
+#pragma unroll
+      for (int e = 0; e < W; ++e) y[e] = x[W * v + e];
+      *reinterpret_cast<vt*>(row + dv) = y;
     } else {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        DK[d + t] = xk[t];
-        DV[d + t] = xv[t];
-      }
+      for (int e = 0; e < W; ++e) row[dv + e] = x[W * v + e];
     }
   }
 }
 
-// dQ (times the softmax scale) of 16 queries from the dQ pass's accumulators:
-// lane (g, c), tile t, register i holds row q0 + row(i, g), d = 4 c + t.
-template <typename T>
-__device__ __forceinline__ void store_q16(const AttnArgs& a, int64_t b, int64_t h, int q0,
-                                          const typename A16<T>::acc_t (&dq)[4], int g, int c) {
-  using M = A16<T>;
-  T* DQ = (T*)a.dq + b * a.sdq.b + h * a.sdq.h + 4 * c;
-  const T scale = (T)a.scale;
+// dK (times the softmax scale) and dV of 16 keys from the key pass's
+// accumulators: lane (g, c), tile t, register i holds key k0 + c,
+// d = N row(i, g) + t.
+template <int DP, bool RAG>
+__device__ __forceinline__ void store_kv16(const AttnArgs& a, int64_t b, int64_t h, int k0, float (&xk)[DP / 16],
+                                           float (&xv)[DP / 16], int i, int g, int c) {
+  constexpr int N = DP / 16;
+  if (RAG && k0 + c >= (int)a.T) return;
+  float* DK = (float*)a.dk + b * a.sdk.b + h * a.sdk.h + (int64_t)(k0 + c) * a.sdk.t;
+  float* DV = (float*)a.dv + b * a.sdv.b + h * a.sdv.h + (int64_t)(k0 + c) * a.sdv.t;
+  const int d = N * A16<float>::row(i, g);
+#pragma unroll
+  for (int t = 0; t < N; ++t) xk[t] *= (float)a.scale;
+  put_row<N, RAG>(DK, d, (int)a.D, xk, a.ovec != 0);
+  put_row<N, RAG>(DV, d, (int)a.D, xv, a.ovec != 0);
+}
+template <int DP, bool RAG>
+__device__ __forceinline__ void store_kv16(const AttnArgs& a, int64_t b, int64_t h, int k0,
+                                           const A16<float>::acc_t (&dk)[DP / 16],
+                                           const A16<float>::acc_t (&dv)[DP / 16], int g, int c) {
+  constexpr int N = DP / 16;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    T* row = DQ + (int64_t)(q0 + M::row(i, g)) * a.sdq.t;
-    const typename M::acc_t x = {dq[0][i] * scale, dq[1][i] * scale, dq[2][i] * scale, dq[3][i] * scale};
-    if (a.ovec) {
+    float xk[N], xv[N];
 #pragma unroll
-      for (int v = 0; v < 4 / M::VEC; ++v) {
-        typename M::vec_t y;
-#pragma unroll
-        for (int e = 0; e < M::VEC; ++e) y[e] = x[M::VEC * v + e];
-        *reinterpret_cast<typename M::vec_t*>(row + M::VEC * v) = y;
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) row[t] = x[t];
+    for (int t = 0; t < N; ++t) {
+      xk[t] = dk[t][i];
+      xv[t] = dv[t][i];
     }
+    store_kv16<DP, RAG>(a, b, h, k0, xk, xv, i, g, c);
   }
 }
 
@@ -1183,31 +1214,39 @@ __host__ __device__ inline int64_t ds16_tiles(int64_t nt) { return nt * (nt + 1)
 // p + nt/2 .. nt - 1), then all of key tile j'. Every wave thus carries nt/2
 // or nt/2 + 1 tile pairs whatever p, and one two-way sum (key tile j's
 // partial dK and dV, wave 0's first) remains.
-// Each lane holds its key's K and V slices in registers; the query tiles'
+// (W = 2.) Each lane holds its key's K and V slices in registers; the query tiles'
 // Q and dO rows pass through the wave's own LDS, the next one prefetched into
 // registers. For each tile pair: S = Q K^T and dP = dO V^T, P recomputed from
 // the forward's row max and sum, dS = P * (dP - rowsum(dO * O)) written to the
 // workspace, dV^T += dO^T P and dK^T += Q^T dS.
-// Aligned float32 path only: D = 64, T a multiple of 32, 16-byte access.
-template <typename T>
-__global__ void __launch_bounds__(128, 3) attn_bwd_kvp_kernel(AttnArgs a) {
-  static_assert(sizeof(T) == 4, "float32 only");
+// W = 4 (D above 64): wave w takes every fourth query tile of either key tile
+// and the four partials are added through LDS after each. The partials lie in
+// the waves' own tile regions, so four waves at DP = 128 take 68 KB and two
+// such blocks share a CU (two waves per SIMD, all that 256 registers allow).
+// Float32 with 16-byte access; the aligned form: D = 64, T a multiple of 32.
+template <int DP, int W, bool RAG>
+__global__ void __launch_bounds__(64 * W, DP == 64 && W == 2 ? 3 : 2) attn_bwd_kvp_kernel(AttnArgs a) {
+  typedef float T;
+  using P = P16<DP>;
   using M = A16<T>;
   typedef typename M::vec_t VT;
   typedef typename M::acc_t AT;
-  constexpr int MT = 16, DP = 64, VEC = M::VEC;
-  constexpr int LD = DP + VEC;                 // padded LDS row
-  constexpr int TILE = MT * LD;
-  constexpr int WAVE_LDS = 2 * TILE + 2 * MT;  // Q rows, dO rows, 2 statistics per row
-  constexpr int NV = MT * DP / VEC / 64;       // 16-byte vectors per lane per tile and operand
-  constexpr int RPV = 64 * VEC / DP;           // rows covered by one vector index
-  constexpr int NF = 16 / VEC;                 // vectors of a lane's 16-element K / V slice
-  constexpr int STASH = 2 * 4 * 4 * 64;        // wave 1's partial dK, dV of key tile j, register order
-  __shared__ __attribute__((aligned(16))) T lds[2 * WAVE_LDS + STASH];
+  constexpr int MT = 16, VEC = M::VEC, N = P::N, SL = P::SL;
+  constexpr int LD = P::LD, TILE = P::TILE;    // padded LDS row
+  constexpr int WAVE_LDS = 2 * TILE + 3 * MT;  // Q rows, dO rows, 2 (RAG: 3) statistics per row
+  constexpr int NV = P::NV;                    // 16-byte vectors per lane per tile and operand
+  constexpr int NF = P::NF;                    // vectors of a lane's K / V slice
+  // partial dK and dV in register order: wave 1's in a place of its own (W = 2),
+  // or every wave's in its own region once its tiles are read (W = 4)
+  constexpr int STASH = 2 * N * 4 * 64;
+  static_assert((W == 2 || W == 4) && STASH <= WAVE_LDS, "partials fit a wave's region");
+  __shared__ __attribute__((aligned(16))) T lds[W * WAVE_LDS + (W == 2 ? STASH : 0)];
 
   const int bh = blockIdx.x;
   const int64_t b = bh / a.H, h = bh % a.H;
-  const int Tn = (int)a.T, nt = Tn / MT, half = nt / 2;
+  const int Tn = (int)a.T, D = (int)a.D;
+  const int half = RAG ? (Tn + 2 * MT - 1) / (2 * MT) : Tn / (2 * MT), nt = 2 * half;
+  const int nq = RAG ? (Tn + MT - 1) / MT : nt;  // tiles with a row below T
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
   const T* Q = (const T*)a.q + b * a.sq.b + h * a.sq.h;
@@ -1220,42 +1259,54 @@ __global__ void __launch_bounds__(128, 3) attn_bwd_kvp_kernel(AttnArgs a) {
   T* DS = (T*)a.ds + (int64_t)bh * ds16_tiles(nt) * (MT * MT);
   const T sl2 = (T)(a.scale * 1.4426950408889634);
   constexpr uint32_t S = sizeof(T);
-  const Rsrc rQ = make_rsrc(Q, (uint64_t)Tn * a.sq.t * S), rG = make_rsrc(G, (uint64_t)Tn * a.sdo.t * S);
-  const Rsrc rK = make_rsrc(K, (uint64_t)Tn * a.sk.t * S), rV = make_rsrc(Vv, (uint64_t)Tn * a.sv.t * S);
+  const Rsrc rQ = rows_rsrc<RAG>(Q, Tn, a.sq.t, D), rG = rows_rsrc<RAG>(G, Tn, a.sdo.t, D);
+  const Rsrc rK = rows_rsrc<RAG>(K, Tn, a.sk.t, D), rV = rows_rsrc<RAG>(Vv, Tn, a.sv.t, D);
   const Rsrc rM = make_rsrc(RM, (uint64_t)Tn * S), rL = make_rsrc(RS, (uint64_t)Tn * S),
              rD = make_rsrc(DR, (uint64_t)Tn * S);
   const Rsrc rS = make_rsrc(DS, (uint64_t)ds16_tiles(nt) * MT * MT * S);
 
   T* Qs = lds + wave * WAVE_LDS;
   T* Gs = Qs + TILE;
-  T* ST = Qs + 2 * TILE;  // [0, 16): max + log2(sum), [16, 32): rowsum(dO * O)
-  T* stash = lds + 2 * WAVE_LDS;
+  // [0, 16): max + log2(sum) (RAG: max), [16, 32): rowsum(dO * O), RAG: [32, 48): 1 / sum
+  T* ST = Qs + 2 * TILE;
 
-  // this lane's share of a tile's loads: vector v is row RPV v + lrow, columns lcol ..
-  const int lrow = lane / (DP / VEC), lcol = (lane % (DP / VEC)) * VEC;
-  const uint32_t vq = (uint32_t)(lrow * a.sq.t + lcol) * S, vg = (uint32_t)(lrow * a.sdo.t + lcol) * S;
+  // this lane's share of a tile's loads: vector v is row RPV (v / NCB) + lrow,
+  // columns CPV (v % NCB) + lcol ..
+  const int lrow = lane / (P::CPV / VEC), lcol = (lane % (P::CPV / VEC)) * VEC;
+  uint32_t vq[P::NCB], vg[P::NCB];
+#pragma unroll
+  for (int u = 0; u < P::NCB; ++u) {
+    const int col = lcol + P::CPV * u;
+    vq[u] = RAG && col >= D ? kOutside : (uint32_t)(lrow * a.sq.t + col) * S;
+    vg[u] = RAG && col >= D ? kOutside : (uint32_t)(lrow * a.sdo.t + col) * S;
+  }
   const uint32_t vs = (uint32_t)c * S;
   VT rq[NV], rg[NV];
   T rm = T(0), rl = T(1), rd = T(0);
+  bool rl_in = true;  // a row past T has a zero sum; its probabilities are 0
   auto fetch = [&](int qs) {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      rq[v] = buf_load_v<VT>(rQ, vq, (uint32_t)((qs + RPV * v) * a.sq.t) * S);
-      rg[v] = buf_load_v<VT>(rG, vg, (uint32_t)((qs + RPV * v) * a.sdo.t) * S);
+      const int row = qs + P::RPV * (v / P::NCB);
+      rq[v] = load_at<RAG, VT>(rQ, vq[v % P::NCB], (uint32_t)(row * a.sq.t) * S);
+      rg[v] = load_at<RAG, VT>(rG, vg[v % P::NCB], (uint32_t)(row * a.sdo.t) * S);
     }
-    rm = buf_load1(rM, vs, (uint32_t)qs * S);
-    rl = buf_load1(rL, vs, (uint32_t)qs * S);
-    rd = buf_load1(rD, vs, (uint32_t)qs * S);
+    const uint32_t so = (uint32_t)qs * S;
+    rm = RAG ? buf_load1(rM, vs + so, 0) : buf_load1(rM, vs, so);
+    rl = RAG ? buf_load1(rL, vs + so, 0) : buf_load1(rL, vs, so);
+    rd = RAG ? buf_load1(rD, vs + so, 0) : buf_load1(rD, vs, so);
+    if (RAG) rl_in = qs + c < Tn;
   };
   auto put = [&]() {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int r = RPV * v + lrow;
-      *reinterpret_cast<VT*>(Qs + r * LD + lcol) = rq[v];
-      *reinterpret_cast<VT*>(Gs + r * LD + lcol) = rg[v];
+      const int r = P::RPV * (v / P::NCB) + lrow, col = P::CPV * (v % P::NCB) + lcol;
+      *reinterpret_cast<VT*>(Qs + r * LD + col) = rq[v];
+      *reinterpret_cast<VT*>(Gs + r * LD + col) = rg[v];
     }
     if (lane < MT) {
-      ST[lane] = rm + log2(rl);
+      ST[lane] = RAG ? rm : rm + log2(rl);
+      if (RAG) ST[2 * MT + lane] = rl_in ? T(1) / rl : T(0);
       ST[MT + lane] = rd;
     }
   };
@@ -1268,49 +1319,62 @@ __global__ void __launch_bounds__(128, 3) attn_bwd_kvp_kernel(AttnArgs a) {
   // pairs p = blockIdx.y, + gridDim.y, ...: more than one when the grid would
   // otherwise run in several rounds of resident blocks
   for (int p = blockIdx.y; p < half; p += gridDim.y) {
-    AT dk[4], dv[4];
-    const int nseg = wave == 0 ? 1 : 2;
+    AT dk[N], dv[N];
+    const int nseg = W == 2 && wave == 0 ? 1 : 2;
     for (int seg = 0; seg < nseg; ++seg) {
       const int j = seg == 0 ? p : nt - 1 - p;
-      const int qa = seg == 1 ? j : (wave == 0 ? p : p + half);
-      const int qb = wave == 0 ? p + half - 1 : nt - 1;
+      const int qa = W == 4 ? j + wave : seg == 1 ? j : (wave == 0 ? p : p + half);
+      int qb = W == 2 && wave == 0 ? p + half - 1 : nt - 1;
+      if (RAG) qb = qb < nq ? qb : nq - 1;
       const int k0 = j * MT;
-      // this lane's key k0 + c: elements 16 g .. 16 g + 15 of its K and V rows
+      // this lane's key k0 + c: elements SL g .. SL g + SL - 1 of its K and V rows
       VT kf[NF], vf[NF];
-      const uint32_t kl = (uint32_t)((k0 + c) * a.sk.t + 16 * g) * S, vl = (uint32_t)((k0 + c) * a.sv.t + 16 * g) * S;
+      const uint32_t kl = (uint32_t)((k0 + c) * a.sk.t + SL * g) * S, vl = (uint32_t)((k0 + c) * a.sv.t + SL * g) * S;
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        kf[f] = buf_load_v<VT>(rK, kl, (uint32_t)(16 * f));
-        vf[f] = buf_load_v<VT>(rV, vl, (uint32_t)(16 * f));
+        const bool in = !RAG || SL * g + VEC * f < D;
+        kf[f] = load_at<RAG, VT>(rK, in ? kl : kOutside, (uint32_t)(16 * f));
+        vf[f] = load_at<RAG, VT>(rV, in ? vl : kOutside, (uint32_t)(16 * f));
       }
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt) dk[dt] = dv[dt] = AT(0);
+      for (int dt = 0; dt < N; ++dt) dk[dt] = dv[dt] = AT(0);
       fetch(qa * MT);
       put();
       drain_vm();  // K and V slices in: the loop's waits then cover only its own prefetch
       wave_sync();
-      for (int qt = qa; qt <= qb; ++qt) {
+      constexpr int DQ = W == 4 ? 4 : 1;  // query tiles from one of the wave's to the next
+      for (int qt = qa; qt <= qb; qt += DQ) {
         const int qs = qt * MT;
-        const bool more = qt < qb;
-        if (more) fetch(qs + MT);
+        const bool more = qt + DQ <= qb;
+        if (more) fetch(qs + DQ * MT);
         // S(r, key) and dP(r, key): rows r = the tile's queries, column c = this lane's key
-        AT s = AT(0), dp = AT(0);
+        // (RAG: each as two chains, its error that of a sum of half the length)
+        AT s = AT(0), dp = AT(0), s1 = AT(0), dp1 = AT(0);
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
-          const VT x = *reinterpret_cast<const VT*>(Qs + c * LD + 16 * g + VEC * f);
-          const VT y = *reinterpret_cast<const VT*>(Gs + c * LD + 16 * g + VEC * f);
+          const VT x = *reinterpret_cast<const VT*>(Qs + c * LD + SL * g + VEC * f);
+          const VT y = *reinterpret_cast<const VT*>(Gs + c * LD + SL * g + VEC * f);
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
-            s = M::mma(x[e], kf[f][e], s);
-            dp = M::mma(y[e], vf[f][e], dp);
+            AT& sc = RAG && f % 2 ? s1 : s;
+            AT& dc = RAG && f % 2 ? dp1 : dp;
+            sc = M::mma(x[e], kf[f][e], sc);
+            dc = M::mma(y[e], vf[f][e], dc);
           }
+        }
+        if constexpr (RAG) {
+          s += s1;
+          dp += dp1;
         }
         auto probs = [&](auto maskc) {
           constexpr bool MASK = decltype(maskc)::value;  // the diagonal tile
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int r = M::row(i, g);
-            T pr = ex2(__builtin_fmaf(s[i], sl2, -ST[r]));
+            // RAG: the forward's own numbers, 2^(score - max) with the score
+            // rounded as there, times 1 / sum: the rounding of max + log2(sum),
+            // a larger number, would be the probabilities' largest error
+            T pr = RAG ? ex2(s[i] * sl2 - ST[r]) * ST[2 * MT + r] : ex2(__builtin_fmaf(s[i], sl2, -ST[r]));
             if constexpr (MASK) pr = c > r ? T(0) : pr;  // key above the query: masked
             s[i] = pr;
             dp[i] = pr * (dp[i] - ST[MT + r]);
@@ -1324,54 +1388,73 @@ __global__ void __launch_bounds__(128, 3) attn_bwd_kvp_kernel(AttnArgs a) {
         const uint32_t tb = (uint32_t)((qt * (qt + 1) / 2 + j) * (MT * MT)) * S;
 #pragma unroll
         for (int i = 0; i < 4; ++i) buf_store1(dp[i], rS, (uint32_t)(M::row(i, g) * MT + c) * S, tb);
-        // dV^T += dO^T P ; dK^T += Q^T dS: result tile t, row r is d = 4 r + t,
+        // dV^T += dO^T P ; dK^T += Q^T dS: result tile t, row r is d = N r + t,
         // column = this lane's key, so a lane's A operands are dO and Q rows
-        // row(i, g), d = 4c .. 4c + 3 (16-byte reads)
+        // row(i, g), d = N c .. N c + N - 1 (vector reads)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = M::row(i, g);
-          VT gv[4 / VEC], qv[4 / VEC];
+          T gv[N], qv[N];
+          lds_row(gv, Gs + r * LD + N * c);
+          lds_row(qv, Qs + r * LD + N * c);
 #pragma unroll
-          for (int v = 0; v < 4 / VEC; ++v) {
-            gv[v] = *reinterpret_cast<const VT*>(Gs + r * LD + 4 * c + VEC * v);
-            qv[v] = *reinterpret_cast<const VT*>(Qs + r * LD + 4 * c + VEC * v);
-          }
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            dv[t] = M::mma(gv[t / VEC][t % VEC], s[i], dv[t]);
-            dk[t] = M::mma(qv[t / VEC][t % VEC], dp[i], dk[t]);
+          for (int t = 0; t < N; ++t) {
+            dv[t] = M::mma(gv[t], s[i], dv[t]);
+            dk[t] = M::mma(qv[t], dp[i], dk[t]);
           }
         }
         wave_sync();
         if (more) put();
         wave_sync();
       }
-      if (wave == 1) {
-        if (seg == 0) {  // key tile j's later query tiles: handed to wave 0
+      T* mine = lds + (W == 2 ? 2 * WAVE_LDS : wave * WAVE_LDS);
+      auto stash = [&]() {
 #pragma unroll
-          for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < N; ++dt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              stash[(dt * 4 + i) * 64 + lane] = dk[dt][i];
-              stash[(16 + dt * 4 + i) * 64 + lane] = dv[dt][i];
-            }
-        } else {
-          store_kv16<T>(a, b, h, k0, dk, dv, g, c);
+          for (int i = 0; i < 4; ++i) {
+            mine[(dt * 4 + i) * 64 + lane] = dk[dt][i];
+            mine[(4 * N + dt * 4 + i) * 64 + lane] = dv[dt][i];
+          }
+      };
+      if constexpr (W == 4) {
+        // the four partials added in wave order, register i by wave i
+        stash();
+        __syncthreads();
+        T xk[N], xv[N];
+#pragma unroll
+        for (int dt = 0; dt < N; ++dt) {
+          xk[dt] = xv[dt] = T(0);
+#pragma unroll
+          for (int w = 0; w < W; ++w) {
+            xk[dt] += lds[w * WAVE_LDS + (dt * 4 + wave) * 64 + lane];
+            xv[dt] += lds[w * WAVE_LDS + (4 * N + dt * 4 + wave) * 64 + lane];
+          }
         }
+        store_kv16<DP, RAG>(a, b, h, k0, xk, xv, wave, g, c);
+        __syncthreads();  // read before the next tiles overwrite them
+      } else if (wave == 1) {
+        if (seg == 1)
+          store_kv16<DP, RAG>(a, b, h, k0, dk, dv, g, c);
+        else  // key tile j's later query tiles: handed to wave 0
+          stash();
       }
     }
-    __syncthreads();  // wave 1's partial of key tile j is in the stash
-    if (wave == 0) {
+    if constexpr (W == 2) {
+      __syncthreads();  // wave 1's partial of key tile j is in the stash
+      if (wave == 0) {
+        const T* part = lds + 2 * WAVE_LDS;
 #pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < N; ++dt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          dk[dt][i] += stash[(dt * 4 + i) * 64 + lane];
-          dv[dt][i] += stash[(16 + dt * 4 + i) * 64 + lane];
-        }
-      store_kv16<T>(a, b, h, p * MT, dk, dv, g, c);
+          for (int i = 0; i < 4; ++i) {
+            dk[dt][i] += part[(dt * 4 + i) * 64 + lane];
+            dv[dt][i] += part[(4 * N + dt * 4 + i) * 64 + lane];
+          }
+        store_kv16<DP, RAG>(a, b, h, p * MT, dk, dv, g, c);
+      }
+      __syncthreads();  // the stash is read before the next pair writes it
     }
-    __syncthreads();  // the stash is read before the next pair writes it
   }
 }
 
@@ -1392,40 +1475,42 @@ __global__ void __launch_bounds__(128, 3) attn_bwd_kvp_kernel(AttnArgs a) {
 // is d = 4 c + t, so that a lane's B operands (a K row, d = 4c + t for its
 // d-tiles t, from LDS), its A operands (a dS row, stored [query][key]) and its
 // dQ rows are vectors.
-template <typename T, int NDT>
+template <int DP, int NDT, bool RAG>
 __global__ void __launch_bounds__(512, 2) attn_bwd_qp_kernel(AttnArgs a) {
-  static_assert(sizeof(T) == 4, "float32 only");
-  static_assert(NDT == 4 || NDT == 2, "d-tiles per wave");
+  typedef float T;
+  constexpr int N = DP / 16;
+  static_assert(NDT == N || NDT == N / 2, "d-tiles per wave");
   using M = A16<T>;
   typedef typename M::vec_t VT;
   typedef typename M::acc_t AT;
-  typedef float HT __attribute__((ext_vector_type(NDT)));
-  constexpr int MT = 16, DP = 64, VEC = M::VEC;
+  constexpr int MT = 16, VEC = M::VEC;
   constexpr int LD = DP + VEC;
   constexpr int KT = 2;                         // key tiles per step
   constexpr int STEP = KT * MT * LD;            // one step's K rows in LDS
   constexpr int NTH = 512;
-  constexpr int KV = KT * MT * DP / VEC / NTH;  // K vectors per thread per step
+  constexpr int KVT = KT * MT * DP / VEC;       // K vectors per step
+  constexpr int KV = (KVT + NTH - 1) / NTH;     // of them per thread
   constexpr int SL = 4 / VEC;                   // vectors of a lane's dS row per tile
-  constexpr int SPLIT = 4 / NDT;                // waves per query tile
-  static_assert(KV * NTH * VEC == KT * MT * DP, "K rows: whole vectors per thread");
+  constexpr int SPLIT = N / NDT;                // waves per query tile
+  constexpr int PPB = 4 / SPLIT;                // query tile pairs per block
   __shared__ __attribute__((aligned(16))) T lds[2 * STEP];
 
   const int bh = blockIdx.x, bq = blockIdx.y;
   const int64_t b = bh / a.H, h = bh % a.H;
-  const int Tn = (int)a.T, nt = Tn / MT, half = nt / 2;
+  const int Tn = (int)a.T, D = (int)a.D;
+  const int half = RAG ? (Tn + 2 * MT - 1) / (2 * MT) : Tn / (2 * MT), nt = 2 * half;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
-  const int i0 = NDT * bq + (wave & 3) / SPLIT;
+  const int i0 = PPB * bq + (wave & 3) / SPLIT;
   const int t0 = ((wave & 3) % SPLIT) * NDT;   // this wave's first d-tile
-  const bool live = i0 < half;
   const int qt = wave < 4 ? i0 : nt - 1 - i0;  // this wave's query tile
-  const int jend = nt - 1 - NDT * bq;          // the block's last key tile (the longest mirror tile)
+  const bool live = i0 < half && (!RAG || qt * MT < Tn);
+  const int jend = nt - 1 - PPB * bq;          // the block's last key tile (the longest mirror tile)
   const int nstep = jend / KT + 1;
   constexpr uint32_t S = sizeof(T);
   const T* K = (const T*)a.k + b * a.sk.b + h * a.sk.h;
   const T* DS = (const T*)a.ds + (int64_t)bh * ds16_tiles(nt) * (MT * MT);
-  const Rsrc rK = make_rsrc(K, (uint64_t)Tn * a.sk.t * S);
+  const Rsrc rK = rows_rsrc<RAG>(K, Tn, a.sk.t, D);
   const Rsrc rS = make_rsrc(DS, (uint64_t)ds16_tiles(nt) * MT * MT * S);
 
   int kro[KV], kco[KV];
@@ -1444,7 +1529,7 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_qp_kernel(AttnArgs a) {
     for (int v = 0; v < KV; ++v) {
       const int row = j0 * MT + kro[v];
       const int rowc = row < (jend + 1) * MT ? row : jend * MT + (kro[v] % MT);
-      rk[v] = buf_load_v<VT>(rK, (uint32_t)kco[v] * S, (uint32_t)(rowc * a.sk.t) * S);
+      rk[v] = load_at<RAG, VT>(rK, RAG && kco[v] >= D ? kOutside : (uint32_t)kco[v] * S, (uint32_t)(rowc * a.sk.t) * S);
     }
 #pragma unroll
     for (int u = 0; u < KT; ++u) {
@@ -1456,15 +1541,21 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_qp_kernel(AttnArgs a) {
   };
   auto put = [&](T* Ks) {
 #pragma unroll
-    for (int v = 0; v < KV; ++v) *reinterpret_cast<VT*>(Ks + kro[v] * LD + kco[v]) = rk[v];
+    for (int v = 0; v < KV; ++v)
+      if (KVT % NTH == 0 || (int)threadIdx.x + NTH * v < KVT) *reinterpret_cast<VT*>(Ks + kro[v] * LD + kco[v]) = rk[v];
 #pragma unroll
     for (int u = 0; u < KT; ++u)
 #pragma unroll
       for (int v = 0; v < SL; ++v) xs[u][v] = nx[u][v];
   };
-  AT dq[NDT];
+  // RAG: a sum for each of a step's two key tiles, so that a sum over all keys
+  // is two chains of half the length
+  constexpr int NS = RAG ? KT : 1;
+  AT dq[NDT], dqs[NS][NDT];
 #pragma unroll
-  for (int t = 0; t < NDT; ++t) dq[t] = AT(0);
+  for (int u = 0; u < NS; ++u)
+#pragma unroll
+    for (int t = 0; t < NDT; ++t) dqs[u][t] = AT(0);
   fetch(0);
   put(lds);
   __syncthreads();
@@ -1476,35 +1567,34 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_qp_kernel(AttnArgs a) {
     for (int u = 0; u < KT; ++u) {
       const int j = KT * it + u;
       if (live && j <= qt) {
-        // dQ(r, d = 4c + t) += sum over the tile's keys of dS(r, key) K(key, d)
-        HT kv[4];
+        // dQ(r, d = N c + t) += sum over the tile's keys of dS(r, key) K(key, d)
+        T kv[4][NDT];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) lds_row(kv[q], Ks + (u * MT + M::row(q, g)) * LD + N * c + t0);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          kv[q] = *reinterpret_cast<const HT*>(Ks + (u * MT + M::row(q, g)) * LD + 4 * c + t0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int t = 0; t < NDT; ++t) dq[t] = M::mma(xs[u][q / VEC][q % VEC], kv[q][t], dq[t]);
+          for (int t = 0; t < NDT; ++t) dqs[u % NS][t] = M::mma(xs[u][q / VEC][q % VEC], kv[q][t], dqs[u % NS][t]);
       }
     }
     if (more) put(lds + ((it + 1) & 1) * STEP);
     __syncthreads();
   }
+#pragma unroll
+  for (int t = 0; t < NDT; ++t) {
+    dq[t] = dqs[0][t];
+    if constexpr (NS == 2) dq[t] += dqs[1][t];
+  }
   if (live) {
-    T* DQ = (T*)a.dq + b * a.sdq.b + h * a.sdq.h + 4 * c + t0;
+    T* DQ = (T*)a.dq + b * a.sdq.b + h * a.sdq.h;
     const T scale = (T)a.scale;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      T* row = DQ + (int64_t)(qt * MT + M::row(i, g)) * a.sdq.t;
-      HT x;
+      const int row = qt * MT + M::row(i, g);
+      T x[NDT];
 #pragma unroll
       for (int t = 0; t < NDT; ++t) x[t] = dq[t][i] * scale;
-      if (a.ovec) {
-        *reinterpret_cast<HT*>(row) = x;
-      } else {
-#pragma unroll
-        for (int t = 0; t < NDT; ++t) row[t] = x[t];
-      }
+      if (!RAG || row < Tn) put_row<NDT, RAG>(DQ + (int64_t)row * a.sdq.t, N * c + t0, D, x, a.ovec != 0);
     }
   }
 }
@@ -1694,7 +1784,7 @@ static int attn_bwd_wide(AttnArgs& a) {
 }
 
 // Forward on 16 x 16 tiles over paired ranges (float32 with 16-byte aligned
-// Q, K and V, D = 64, T a multiple of 32): block (bh, p), one wave, query
+// Q, K and V): block (bh, p), W waves, query
 // tile p and then its mirror nt - 1 - p, which see p + 1 and nt - p key
 // tiles, nt + 1 in all, so every wave carries the same work (then the pairs
 // p + gridDim.y, ... when the grid is shortened to one round of resident
@@ -1703,21 +1793,31 @@ static int attn_bwd_wide(AttnArgs& a) {
 // lane's Q slice (its query c, d = 16 g .. 16 g + 15, times scale * log2(e))
 // in registers; P feeds O^T += V^T P^T from registers; the next key tile's K
 // and V rows are prefetched into registers while the current one is computed.
-// Lazy rescaling against a reference max as in attn_fwd_kernel.
-__global__ void __launch_bounds__(64) attn_fwd_p16_kernel(AttnArgs a) {
+// Lazy rescaling against a reference max as in attn_fwd_kernel. With W > 1 the
+// waves take the key tiles in turn, each against a reference of its own, and
+// join their sums through LDS at the end of a query tile: a few heads of a long
+// sequence are too few pairs to fill the chip with one wave each, and the
+// chain of dependent MFMAs per query is W times shorter. At DP = 128 a wave
+// needs 220 to 256 registers, two per SIMD.
+template <int DP, int W, bool RAG>
+__global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(AttnArgs a) {
   using M = A16<float>;
   typedef M::vec_t VT;
   typedef M::acc_t AT;
-  constexpr int MT = 16, DP = 64, VEC = 4, LD = DP + VEC, TILE = MT * LD;
-  constexpr int NV = MT * DP / VEC / 64;  // 16-byte vectors per lane per tile and operand
-  constexpr int RPV = 64 * VEC / DP;      // rows per vector index
-  constexpr int NF = 16 / VEC;            // vectors of a lane's 16-element Q slice
-  __shared__ __attribute__((aligned(16))) float lds[2 * TILE];
-  float* Ks = lds;
-  float* Vs = lds + TILE;
+  using P = P16<DP>;
+  constexpr int MT = 16, VEC = 4, LD = P::LD, TILE = P::TILE, N = P::N, SL = P::SL;
+  constexpr int NV = P::NV;  // 16-byte vectors per lane per tile and operand
+  constexpr int NF = P::NF;  // vectors of a lane's Q slice
+  static_assert(W == 1 || (4 % W == 0 && (4 * N + 2) * 64 <= 2 * TILE), "partials fit a wave's tiles");
+  __shared__ __attribute__((aligned(16))) float lds[W * 2 * TILE];
+  const int wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float* Ks = lds + wave * 2 * TILE;
+  float* Vs = Ks + TILE;
+  __shared__ float tops[W][MT];  // W > 1: the waves' true maxima per query
   const int bh = blockIdx.x;
   const int64_t b = bh / a.H, h = bh % a.H;
-  const int Tn = (int)a.T, nt = Tn / MT;
+  const int Tn = (int)a.T, D = (int)a.D;
+  const int nt = RAG ? 2 * ((Tn + 2 * MT - 1) / (2 * MT)) : Tn / MT;
   const int lane = threadIdx.x & 63;
   const int g = lane >> 4, c = lane & 15;
   const float* Q = (const float*)a.q + b * a.sq.b + h * a.sq.h;
@@ -1726,23 +1826,30 @@ __global__ void __launch_bounds__(64) attn_fwd_p16_kernel(AttnArgs a) {
   float* O = (float*)a.out + b * a.so.b + h * a.so.h;
   const float sl2 = (float)(a.scale * 1.4426950408889634);
   constexpr uint32_t S = 4;
-  const Rsrc rK = make_rsrc(K, (uint64_t)Tn * a.sk.t * S), rV = make_rsrc(V, (uint64_t)Tn * a.sv.t * S);
-  const int lrow = lane / (DP / VEC), lcol = (lane % (DP / VEC)) * VEC;
-  const uint32_t vk = (uint32_t)(lrow * a.sk.t + lcol) * S, vv = (uint32_t)(lrow * a.sv.t + lcol) * S;
+  const Rsrc rK = rows_rsrc<RAG>(K, Tn, a.sk.t, D), rV = rows_rsrc<RAG>(V, Tn, a.sv.t, D);
+  const int lrow = lane / (P::CPV / VEC), lcol = (lane % (P::CPV / VEC)) * VEC;
+  uint32_t vk[P::NCB], vv[P::NCB];
+#pragma unroll
+  for (int u = 0; u < P::NCB; ++u) {
+    const int col = lcol + P::CPV * u;
+    vk[u] = RAG && col >= D ? kOutside : (uint32_t)(lrow * a.sk.t + col) * S;
+    vv[u] = RAG && col >= D ? kOutside : (uint32_t)(lrow * a.sv.t + col) * S;
+  }
   VT rk[NV], rv[NV];
   auto fetch = [&](int j) {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      rk[v] = buf_load_v<VT>(rK, vk, (uint32_t)((j * MT + RPV * v) * a.sk.t) * S);
-      rv[v] = buf_load_v<VT>(rV, vv, (uint32_t)((j * MT + RPV * v) * a.sv.t) * S);
+      const int row = j * MT + P::RPV * (v / P::NCB);
+      rk[v] = load_at<RAG, VT>(rK, vk[v % P::NCB], (uint32_t)(row * a.sk.t) * S);
+      rv[v] = load_at<RAG, VT>(rV, vv[v % P::NCB], (uint32_t)(row * a.sv.t) * S);
     }
   };
   auto put = [&]() {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const int r = RPV * v + lrow;
-      *reinterpret_cast<VT*>(Ks + r * LD + lcol) = rk[v];
-      *reinterpret_cast<VT*>(Vs + r * LD + lcol) = rv[v];
+      const int r = P::RPV * (v / P::NCB) + lrow, col = P::CPV * (v % P::NCB) + lcol;
+      *reinterpret_cast<VT*>(Ks + r * LD + col) = rk[v];
+      *reinterpret_cast<VT*>(Vs + r * LD + col) = rv[v];
     }
   };
   auto wave_sync = [] {
@@ -1760,29 +1867,40 @@ __global__ void __launch_bounds__(64) attn_fwd_p16_kernel(AttnArgs a) {
   for (int seg = 0; seg < 2; ++seg) {
     const int qt = seg == 0 ? p : nt - 1 - p;
     const int q0 = qt * MT;
+    if (RAG && q0 >= Tn) continue;  // the mirror of tile 0, when T's last tile is an even one
     VT qf[NF];
-    const float* qrow = Q + (int64_t)(q0 + c) * a.sq.t + 16 * g;
+    // a query past T reads query T - 1 (its result is not stored)
+    const float* qrow = Q + (int64_t)(RAG && q0 + c >= Tn ? Tn - 1 : q0 + c) * a.sq.t + SL * g;
 #pragma unroll
-    for (int f = 0; f < NF; ++f) qf[f] = *reinterpret_cast<const VT*>(qrow + VEC * f) * sl2;
-    AT o[4];
+    for (int f = 0; f < NF; ++f) {
+      const bool in = !RAG || SL * g + VEC * f < D;
+      const VT x = *reinterpret_cast<const VT*>(in ? qrow + VEC * f : Q);
+      qf[f] = in ? (RAG ? x : x * sl2) : VT(0);
+    }
+    AT o[N];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) o[t] = AT(0);
+    for (int t = 0; t < N; ++t) o[t] = AT(0);
     float mref = -INFINITY, mtop = -INFINITY, l = 0.f;
-    fetch(0);
+    fetch(wave);
     put();
     drain_vm();
     wave_sync();
-    for (int j = 0; j <= qt; ++j) {
-      const bool more = j < qt;
-      if (more) fetch(j + 1);
+    for (int j = wave; j <= qt; j += W) {
+      const bool more = j + W <= qt;
+      if (more) fetch(j + W);
       // S^T(key 4g + i, query c) in base-2 units
-      AT s = AT(0);
+      // (RAG: two chains, as in the key pass)
+      AT s = AT(0), s1 = AT(0);
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        const VT x = *reinterpret_cast<const VT*>(Ks + c * LD + 16 * g + VEC * f);
+        const VT x = *reinterpret_cast<const VT*>(Ks + c * LD + SL * g + VEC * f);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) s = M::mma(x[e], qf[f][e], s);
+        for (int e = 0; e < VEC; ++e) {
+          AT& sc = RAG && f % 2 ? s1 : s;
+          sc = M::mma(x[e], qf[f][e], sc);
+        }
       }
+      if constexpr (RAG) s = (s + s1) * sl2;  // one rounding per score instead of one per term
       if (j == qt) {  // the diagonal tile: keys after the query masked
 #pragma unroll
         for (int i = 0; i < 4; ++i) s[i] = 4 * g + i > c ? -INFINITY : s[i];
@@ -1794,7 +1912,7 @@ __global__ void __launch_bounds__(64) attn_fwd_p16_kernel(AttnArgs a) {
         const float alpha = ex2(mref - mnew);  // mref = -inf on the first tile: 0
         l *= alpha;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] *= alpha;
+        for (int t = 0; t < N; ++t) o[t] *= alpha;
         mref = mnew;
       }
 #pragma unroll
@@ -1802,12 +1920,13 @@ __global__ void __launch_bounds__(64) attn_fwd_p16_kernel(AttnArgs a) {
         s[i] = ex2(s[i] - mref);
         l += s[i];
       }
-      // O^T(d = 4 m + t, query c) += sum over the tile's keys of V(key, d) P(key, query)
+      // O^T(d = N m + t, query c) += sum over the tile's keys of V(key, d) P(key, query)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const VT vr = *reinterpret_cast<const VT*>(Vs + (4 * g + i) * LD + 4 * c);
+        float vr[N];
+        lds_row(vr, Vs + (4 * g + i) * LD + N * c);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = M::mma(vr[t], s[i], o[t]);
+        for (int t = 0; t < N; ++t) o[t] = M::mma(vr[t], s[i], o[t]);
       }
       wave_sync();
       if (more) put();
@@ -1816,22 +1935,60 @@ __global__ void __launch_bounds__(64) attn_fwd_p16_kernel(AttnArgs a) {
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     mtop = gmax(mtop);
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    // lane (g, c) register i of tile t: d = 4 (4 g + i) + t of query c
-    float* orow = O + (int64_t)(q0 + c) * a.so.t + 16 * g;
+    if constexpr (W > 1) {
+      // the waves' outputs and sums against the largest of their reference
+      // maxima (a wave without a key tile: -inf, weight 0), added in wave
+      // order; wave w finishes registers w, w + W, ...
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const VT x = {o[0][i] * inv, o[1][i] * inv, o[2][i] * inv, o[3][i] * inv};
-      if (a.ovec) {
-        *reinterpret_cast<VT*>(orow + 4 * i) = x;
-      } else {  // O not 16-byte aligned: element stores, same values
+      for (int t = 0; t < N; ++t)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) orow[4 * i + t] = x[t];
+        for (int i = 0; i < 4; ++i) Ks[(t * 4 + i) * 64 + lane] = o[t][i];
+      Ks[4 * N * 64 + lane] = mref;
+      Ks[(4 * N + 1) * 64 + lane] = l;
+      if (lane < MT) tops[wave][lane] = mtop;
+      __syncthreads();
+      float wt[W], mall = -INFINITY;
+      mtop = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        mall = fmaxf(mall, lds[w * 2 * TILE + 4 * N * 64 + lane]);
+        mtop = fmaxf(mtop, tops[w][c]);
       }
+      l = 0.f;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const float mw = lds[w * 2 * TILE + 4 * N * 64 + lane];
+        wt[w] = mw == mall ? 1.f : ex2(mw - mall);
+        l += lds[w * 2 * TILE + (4 * N + 1) * 64 + lane] * wt[w];
+      }
+      mref = mall;
+#pragma unroll
+      for (int t = 0; t < N; ++t)
+#pragma unroll
+        for (int u = 0; u < 4 / W; ++u) {
+          const int i = wave + W * u;
+          float x = 0.f;
+#pragma unroll
+          for (int w = 0; w < W; ++w) x += lds[w * 2 * TILE + (t * 4 + i) * 64 + lane] * wt[w];
+          o[t][u] = x;
+        }
+      __syncthreads();  // read before the next segment's tiles overwrite them
     }
-    if (g == 0) {
-      ((float*)a.rowmax)[(int64_t)bh * Tn + q0 + c] = mtop;
-      ((float*)a.rowsum)[(int64_t)bh * Tn + q0 + c] = l * ex2(mref - mtop);
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    // lane (g, c) register i of tile t: d = N (4 g + i) + t of query c
+    if (!RAG || q0 + c < Tn) {
+      float* orow = O + (int64_t)(q0 + c) * a.so.t;
+#pragma unroll
+      for (int u = 0; u < 4 / W; ++u) {
+        float x[N];
+#pragma unroll
+        for (int t = 0; t < N; ++t) x[t] = o[t][u] * inv;
+        put_row<N, RAG>(orow, N * (4 * g + wave + W * u), D, x, a.ovec != 0);
+      }
+      if (g == 0 && wave == 0) {
+        ((float*)a.rowmax)[(int64_t)bh * Tn + q0 + c] = mtop;
+        ((float*)a.rowsum)[(int64_t)bh * Tn + q0 + c] = l * ex2(mref - mtop);
+      }
     }
     wave_sync();  // the last tile's rows are read before the next segment's put
   }
@@ -1867,25 +2024,74 @@ static int resident_blocks(F kernel, int threads) {
   return n;
 }
 
+// The paired-range kernels on 16 x 16 tiles take float32 with 16-byte access:
+// D = 64 with T a multiple of 32 without bounds (1), and D = 36 .. 128 with any
+// T where rows and columns outside read as zero through the buffers' bounds
+// (2): that needs rows that do not overlap and extents below 2^31 bytes. 0:
+// none of these. Against the 128-row blocks of attn_fwd_kernel and
+// attn_bwd_kv_kernel, whose longest block walks the whole sequence by itself
+// (D up to 64), and against materialised scores (D above 64), forward and
+// backward: B 5, H 12, T 499, D 64 225 -> 100 us, B 2, H 8, T 2000, D 128
+// 1490 -> 565 us, with smaller errors against float64 (dK at these: 5.7e-7 ->
+// 4.1e-7, 6.3e-7 -> 5.8e-7).
+// Waves per block and pair (a constant of the form, so that a (batch, head)
+// has the same bits in any batch): forward 1 (form 1), 2 (D up to 64: B 5,
+// H 12, T 499 forward 35 us with one, 31 with two, 37 with four) or 4 (above:
+// B 2, H 8, T 777, D 96 63, 55 and 37 us with one, two and four; 8, 8, 1000,
+// 128 166, 169 and 189); key pass 2 (up to 64: 68 us, 74 with four, at 5, 12,
+// 499) or 4 (above: 92 us, 120 with two, at 2, 8, 777, 96; and sums of a
+// quarter of the sequence keep the error of split products).
+template <typename T>
+static int paired_form(const AttnArgs& a, bool backward) {
+  if (sizeof(T) != 4 || !a.vec) return 0;
+  if (a.D == 64 && a.T % 32 == 0) return 1;
+  if (a.D <= 32 || a.D > 128) return 0;
+  const Strides3* st[] = {&a.sq, &a.sk, &a.sv, &a.sdo};
+  for (int i = 0; i < (backward ? 4 : 3); ++i)
+    if (st[i]->t < a.D || st[i]->t >= ((int64_t)1 << 29) / (a.T + 64)) return 0;
+  return a.T < (1 << 15) ? 2 : 0;  // dS of one (batch, head) below 2^31 bytes too
+}
+
+template <int DP, int W, bool RAG>
+static int attn_fwd_paired(AttnArgs& a) {
+  static const int resident = resident_blocks(attn_fwd_p16_kernel<DP, W, RAG>, 64 * W);
+  const unsigned pairs = (unsigned)cdiv(a.T, 32);
+  const unsigned per = pairs_per_block(a.B * a.H, pairs, resident);
+  attn_fwd_p16_kernel<DP, W, RAG><<<dim3((unsigned)(a.B * a.H), (unsigned)cdiv(pairs, per)), 64 * W, 0, stream()>>>(a);
+  LAUNCH_CHECK("attn_fwd_p16_kernel");
+  return DTMI_OK;
+}
+
+template <int DP, int W, bool RAG>
+static void attn_bwd_paired(AttnArgs& a) {
+  constexpr int N = DP / 16;
+  // DP = 96: three d-tiles per wave would not be vectors, so no split there
+  constexpr int NHALF = N % 4 == 0 ? N / 2 : N;
+  const unsigned pairs = (unsigned)cdiv(a.T, 32), bh = (unsigned)(a.B * a.H);
+  static const int resident = resident_blocks(attn_bwd_kvp_kernel<DP, W, RAG>, 64 * W);
+  const unsigned per = pairs_per_block(bh, pairs, resident);
+  attn_bwd_kvp_kernel<DP, W, RAG><<<dim3(bh, (unsigned)cdiv(pairs, per)), 64 * W, 0, stream()>>>(a);
+  // fewer than two four-pair blocks per CU: split the d-tiles instead
+  if (NHALF != N && (int64_t)bh * cdiv(pairs, 4) < 2 * (int64_t)num_cus())
+    attn_bwd_qp_kernel<DP, NHALF, RAG><<<dim3(bh, (unsigned)cdiv(pairs, 2)), 512, 0, stream()>>>(a);
+  else
+    attn_bwd_qp_kernel<DP, N, RAG><<<dim3(bh, (unsigned)cdiv(pairs, 4)), 512, 0, stream()>>>(a);
+}
+
 template <typename T>
 static int attn_fwd_impl(AttnArgs& a) {
   constexpr int MT = AM<T>::MT;
   const int dp = pick_dp<T>(a.D);
-  if (dp < 0) return attn_fwd_wide<T>(a);
+  const int form = paired_form<T>(a, false);
+  if (dp < 0 && !form) return attn_fwd_wide<T>(a);
   dim3 grid((unsigned)cdiv(a.T, 4 * MT), (unsigned)(a.B * a.H));
   // causal-exact FLOP: 2 GEMMs of 2*D*T(T+1)/2 per (b, h)
   TimedLaunch tl(DTMI_FAM_ATTN_FWD, 2.0 * 2.0 * a.B * a.H * a.D * (double)a.T * (a.T + 1) / 2.0);
-  if constexpr (std::is_same<T, float>::value) {
-    // D = 64, T a multiple of 32, 16-byte reads of Q, K and V: the
-    // paired-range forward on 16 x 16 tiles (O aligned or not, same bits)
-    if (a.vec && a.D == 64 && a.T % 32 == 0) {
-      static const int resident = resident_blocks(attn_fwd_p16_kernel, 64);
-      const unsigned pairs = (unsigned)(a.T / 32);
-      const unsigned per = pairs_per_block(a.B * a.H, pairs, resident);
-      attn_fwd_p16_kernel<<<dim3((unsigned)(a.B * a.H), (unsigned)cdiv(pairs, per)), 64, 0, stream()>>>(a);
-      LAUNCH_CHECK("attn_fwd_p16_kernel");
-      return DTMI_OK;
-    }
+  if (form == 1) return attn_fwd_paired<64, 1, false>(a);
+  if (form == 2) {
+    if (a.D <= 64) return attn_fwd_paired<64, 2, true>(a);
+    if (a.D <= 96) return attn_fwd_paired<96, 4, true>(a);
+    return attn_fwd_paired<128, 4, true>(a);
   }
   DP_SWITCH(dp, attn_fwd_kernel, T, grid)
   LAUNCH_CHECK("attn_fwd_kernel");
@@ -1901,23 +2107,23 @@ template <typename T>
 static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
   constexpr int MT = AM<T>::MT;
   const int dp = pick_dp<T>(a.D);
-  if (dp < 0) return attn_bwd_wide<T>(a);
+  int form = paired_form<T>(a, true);
+  // dS for the dQ pass: B*H*T*T elements (the causal tiles only on the
+  // paired-range path), up to g_max_ds_bytes; beyond that the dQ pass
+  // recomputes S, P and dP itself, or (D above 64) the scores of one batch
+  // element are materialised.
+  a.ds = nullptr;
+  const double ds_bytes = form ? (double)a.B * a.H * (double)ds16_tiles(2 * cdiv(a.T, 32)) * 256.0 * sizeof(T)
+                               : (double)a.B * a.H * a.T * a.T * sizeof(T);
+  const bool keep_ds = ds_bytes <= (double)g_max_ds_bytes;
+  if (!keep_ds) form = 0;
+  if (dp < 0 && !form) return attn_bwd_wide<T>(a);
   const int64_t rows = a.B * a.H * a.T;
   void* drow = nullptr;  // rowsum(dO * O): given, or computed below
   int rc = drow_in ? 0 : pool_alloc(&drow, (size_t)rows * sizeof(T));
   if (rc) return rc;
   a.drow = drow_in ? const_cast<void*>(drow_in) : drow;
-  // float32, D = 64, T a multiple of 32, 16-byte access: the paired-range
-  // kernels on 16 x 16 tiles, with dS in causal tiles (float64 keeps the
-  // 64-key blocks: its key pass needs twice the registers)
-  const bool pair16 = std::is_same<T, float>::value && a.vec && a.D == 64 && a.T % 32 == 0;
-  // dS for the dQ pass: B*H*T*T elements (the causal tiles only on the
-  // paired-range path), up to g_max_ds_bytes; beyond that the dQ pass
-  // recomputes S, P and dP itself.
-  a.ds = nullptr;
-  const double ds_bytes = pair16 ? (double)a.B * a.H * (double)ds16_tiles(a.T / 16) * 256.0 * sizeof(T)
-                                 : (double)a.B * a.H * a.T * a.T * sizeof(T);
-  if (ds_bytes <= (double)g_max_ds_bytes) {
+  if (keep_ds) {
     rc = pool_alloc(&a.ds, (size_t)ds_bytes);
     if (rc) {
       pool_free(drow);
@@ -1937,18 +2143,15 @@ static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
       attn_drow_kernel<T><<<(unsigned)cdiv(rows, 4), 256, 0, stream()>>>(a);
     }
     dim3 grid((unsigned)cdiv(a.T, 4 * MT), (unsigned)(a.B * a.H));
-    if (pair16 && a.ds) {
-      if constexpr (std::is_same<T, float>::value) {
-        const unsigned pairs = (unsigned)(a.T / 32);
-        static const int resident = resident_blocks(attn_bwd_kvp_kernel<float>, 128);
-        const unsigned per = pairs_per_block(a.B * a.H, pairs, resident);
-        attn_bwd_kvp_kernel<T><<<dim3((unsigned)(a.B * a.H), (unsigned)cdiv(pairs, per)), 128, 0, stream()>>>(a);
-        // fewer than two four-pair blocks per CU: split the d-tiles instead
-        if ((int64_t)a.B * a.H * cdiv(pairs, 4) < 2 * (int64_t)num_cus())
-          attn_bwd_qp_kernel<T, 2><<<dim3((unsigned)(a.B * a.H), (unsigned)cdiv(pairs, 2)), 512, 0, stream()>>>(a);
-        else
-          attn_bwd_qp_kernel<T, 4><<<dim3((unsigned)(a.B * a.H), (unsigned)cdiv(pairs, 4)), 512, 0, stream()>>>(a);
-      }
+    if (form == 1) {
+      attn_bwd_paired<64, 2, false>(a);
+    } else if (form == 2) {
+      if (a.D <= 64)
+        attn_bwd_paired<64, 2, true>(a);
+      else if (a.D <= 96)
+        attn_bwd_paired<96, 4, true>(a);
+      else
+        attn_bwd_paired<128, 4, true>(a);
     } else {
       // 128-key (128-query) blocks; the dQ pass reads dS, or recomputes it
       // above the workspace bound

@@ -309,3 +309,45 @@ def test_results_written_through_unaligned_views(dev, dt, shape):
     assert rel_err(o2.numpy(), o_ref) <= TOL[dt]
     for a, r in zip(grads2, ref):
         assert rel_err(a.numpy(), r) <= TOL[dt]
+
+
+@pytest.mark.parametrize("D_", [36, 64, 80, 96, 100, 128])
+@pytest.mark.parametrize("T", [1, 15, 17, 33, 49, 97, 130, 257])
+def test_paired_ranges_at_ragged_lengths_and_other_head_dimensions(dev, T, D_):
+    """The paired-range kernels where T is no multiple of 32 and D is not 64
+    (a last query tile that is partly or wholly past T, columns past D, padded
+    widths 64, 96 and 128), on strided q, k and v of a [B, T, 3, H, D]
+    projection. Batch element 1 is NaN throughout, so a row or column read
+    past the end of batch element 0 shows in its results; what lies between
+    and after the written gradients keeps its value. Oracle and bar as above."""
+    D, K = _dev()
+    H = 3
+    rng = np.random.default_rng(T * 131 + D_)
+    qkv = np.full((2, T, 3, H, D_), np.nan, np.float32)
+    qkv[0] = rng.standard_normal((T, 3, H, D_))
+    g = np.full((2, T, H, D_), np.nan, np.float32)
+    g[0] = rng.standard_normal((T, H, D_))
+    q, k, v = (np.ascontiguousarray(qkv[:1, :, i].transpose(0, 2, 1, 3)) for i in range(3))
+    gh = np.ascontiguousarray(g[:1].transpose(0, 2, 1, 3))
+    o_ref, p, scale = ops.attention_fwd(q, k, v)
+    refs = ops.attention_bwd(gh, q, k, v, p, scale)
+    t5 = D.from_numpy(qkv).transpose(2, 0, 3, 1, 4)
+    obuf = D.full((T + 1, 2, H, D_), 7.0, np.float32)
+    ov = obuf[:T].transpose(1, 2, 0, 3)
+    _, rmax, rsum = K.attn_fwd(t5[0], t5[1], t5[2], out=ov)
+    dbuf = D.full((T + 1, 2, 3, H, D_), 7.0, np.float32)
+    d5 = dbuf[:T].transpose(2, 1, 3, 0, 4)
+    K.attn_bwd(t5[0], t5[1], t5[2], ov, D.from_numpy(g).transpose(0, 2, 1, 3), rmax, rsum,
+               dq=d5[0], dk=d5[1], dv=d5[2])
+    go, gd = obuf.numpy(), dbuf.numpy()
+    tol = TOL[np.float32]
+    assert rel_err(go[:T, :1].transpose(1, 2, 0, 3), o_ref) <= tol
+    m_ref, l_ref = ops.row_stats(q, k)
+    assert rel_err(rmax.numpy()[:1], m_ref * np.log2(np.e)) <= tol
+    assert rel_err(rsum.numpy()[:1], l_ref) <= tol
+    for i, ref in enumerate(refs):
+        if T == 1 and i < 2:  # one key: dQ and dK are 0, what is left is rounding of dP - rowsum(dO * O)
+            assert np.max(np.abs(gd[:T, 0, i])) <= tol
+        else:
+            assert rel_err(gd[:T, :1, i].transpose(1, 2, 0, 3), ref) <= tol
+    assert np.all(go[T:] == 7.0) and np.all(gd[T:] == 7.0)
