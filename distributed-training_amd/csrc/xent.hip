@@ -158,7 +158,11 @@ __global__ void __launch_bounds__(256) xent_bwd_kernel(T* __restrict__ dz, const
 // xent_grad_scale_kernel rescales in place when the upstream gradient is not
 // 1. Max and sum are combined in a fixed order: a butterfly per wave, then
 // the 16 wave results in wave order.
-template <int NV>
+// RAG: any V. Rows then start at any multiple of 4 bytes: the up to three
+// logits before a row's first 16-byte boundary and after its last are one each
+// for the first threads. At 4096 x 50257 the two-kernel form took 675 us with
+// its 4-byte accesses, this 335 (4.9 TB/s, a large copy's rate).
+template <int NV, bool RAG>
 __global__ void __launch_bounds__(1024) xent_fused_kernel(float* __restrict__ dz, float* __restrict__ rowmax,
                                                            float* __restrict__ rowsum, float* __restrict__ logp_t,
                                                            const float* __restrict__ z,
@@ -167,12 +171,21 @@ __global__ void __launch_bounds__(1024) xent_fused_kernel(float* __restrict__ dz
   typedef float f4 __attribute__((ext_vector_type(4)));
   __shared__ float red[16];
   const int64_t row = blockIdx.x;
-  const f4* zr = reinterpret_cast<const f4*>(z + row * V);
-  f4* dr = reinterpret_cast<f4*>(dz + row * V);
-  const int nv = (int)(V / 4);
+  const int lead = RAG ? (int)((4 - (row * V) % 4) % 4) : 0;  // V > 3 here
+  const f4* zr = reinterpret_cast<const f4*>(z + row * V + lead);
+  f4* dr = reinterpret_cast<f4*>(dz + row * V + lead);
+  const int nv = (int)((V - lead) / 4);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   f4 v[NV];
   float m = -INFINITY;
+  // the logit outside the vectors that this thread has, if any
+  int ei = -1;
+  float ve = 0.f;
+  if constexpr (RAG) {
+    if (tid < lead) ei = tid;
+    if (tid >= 4 && lead + 4 * nv + tid - 4 < (int)V) ei = lead + 4 * nv + tid - 4;
+    if (ei >= 0) m = ve = z[row * V + ei];
+  }
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int i = tid + 1024 * j;
@@ -190,6 +203,10 @@ __global__ void __launch_bounds__(1024) xent_fused_kernel(float* __restrict__ dz
   __syncthreads();
   // v becomes exp(z - max) (0 past the row end), reused by the gradient
   float sl = 0.f;
+  if (RAG && ei >= 0) {
+    ve = expf(ve - M);
+    sl = ve;
+  }
 #pragma unroll
   for (int j = 0; j < NV; ++j)
 #pragma unroll
@@ -224,13 +241,20 @@ __global__ void __launch_bounds__(1024) xent_fused_kernel(float* __restrict__ dz
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float p = v[j][e] * rS;
-        if (4 * i + e == t32) p = p - 1.f;
+        if (lead + 4 * i + e == t32) p = p - 1.f;
         o[e] = p * inv_n;
       }
       dr[i] = o;
     }
   }
+  if (RAG && ei >= 0) {
+    float p = ve * rS;
+    if (ei == t32) p = p - 1.f;
+    dz[row * V + ei] = p * inv_n;
+  }
 }
+
+constexpr int64_t kFusedRagged = 1024;  // see dtmi_xent_fused
 
 // x *= g[0] unless g[0] == 1 (then x is already the gradient).
 template <typename T>
@@ -327,8 +351,13 @@ DTMI_EXPORT int dtmi_xent_fused(int dtype, void* loss, void* dlogits, void* rowm
              (long long)rows, (long long)vocab);
   DTMI_CHECK(loss && dlogits && rowmax && rowsum && logits && targets, "dtmi_xent_fused: NULL pointer");
   const int64_t nv = vocab / 4;
-  const bool fused = dtype == DTMI_F32 && vocab % 4 == 0 && nv <= 16 * 1024 && aligned(logits, 16) &&
-                     aligned(dlogits, 16);
+  // A vocabulary that is no multiple of 4 takes the one-pass form above 1024
+  // logits: 2048 x 20001 119 -> 94 us, 2048 x 4099 31 -> 22, 1024 x 2049
+  // 19.7 -> 16.9, 2048 x 1027 level; below, a row leaves most of its block
+  // without a vector (4096 x 65 19 us with two kernels, 31 with one).
+  const bool rag = vocab % 4 != 0;
+  const bool fused = dtype == DTMI_F32 && nv <= 16 * 1024 && aligned(logits, 16) && aligned(dlogits, 16) &&
+                     (!rag || vocab > kFusedRagged);
   if (!fused) {  // the two-kernel form: forward, then the gradient for an upstream gradient of 1
     int rc = dtmi_xent_fwd(dtype, loss, rowmax, rowsum, logits, targets, rows, vocab);
     if (rc) return rc;
@@ -342,8 +371,12 @@ DTMI_EXPORT int dtmi_xent_fused(int dtype, void* loss, void* dlogits, void* rowm
     const float inv_n = 1.f / (float)rows;
     auto go = [&](auto nvc) {
       constexpr int NV = decltype(nvc)::value;
-      xent_fused_kernel<NV><<<(unsigned)rows, 1024, 0, stream()>>>((float*)dlogits, (float*)rowmax, (float*)rowsum,
-                                                                   logp, (const float*)logits, targets, vocab, inv_n);
+      if (rag)
+        xent_fused_kernel<NV, true><<<(unsigned)rows, 1024, 0, stream()>>>(
+            (float*)dlogits, (float*)rowmax, (float*)rowsum, logp, (const float*)logits, targets, vocab, inv_n);
+      else
+        xent_fused_kernel<NV, false><<<(unsigned)rows, 1024, 0, stream()>>>(
+            (float*)dlogits, (float*)rowmax, (float*)rowsum, logp, (const float*)logits, targets, vocab, inv_n);
     };
     const int need = (int)cdiv(nv, 1024);
     if (need <= 1)

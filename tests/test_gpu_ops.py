@@ -173,6 +173,30 @@ def test_cross_entropy_single_pass_forward_and_gradient(dev, dt, rows, V):
     assert rel_err(K.xent_bwd(dz, dtgt, rmax, rsum, g_host=1.0).numpy(), g1) <= TOL[dt]
 
 
+@pytest.mark.parametrize("V", [1025, 1026, 1027, 4099, 50257, 65533, 65539])
+def test_cross_entropy_single_pass_with_rows_off_the_16_byte_grid(dev, V):
+    """Vocabularies that are no multiple of 4: rows start 0 to 3 logits off a
+    16-byte boundary, and a row's first and last logits lie outside its
+    vectors; targets and the row's maximum among those too, up to the one-pass
+    form's longest row. Loss and gradient against the oracle."""
+    D, K = _dev()
+    rng = np.random.default_rng(V)
+    z = (rng.standard_normal((9, V)) * 3).astype(np.float32)
+    t = np.array([0, V - 1, 1, V - 2, 2, V - 3, 3, V // 2, V - 4])
+    for r, j in enumerate((0, 1, V - 1, V - 2, 2, 0, V - 3, V - 1, 5)):
+        z[r, j] = 20.0
+    loss, cache = ops.cross_entropy_fwd(z, t)
+    g = ops.cross_entropy_bwd(np.asarray(1.0, dtype=np.float32), z, t, cache)
+    dloss, _, _, dl = K.xent_fused(D.from_numpy(z), D.from_numpy(t.astype(np.int64)))
+    assert rel_err(dloss.numpy(), loss) <= TOL[np.float32]
+    got = dl.numpy()
+    assert rel_err(got, g) <= TOL[np.float32]
+    # every entry by itself, (p - [target]) / rows with p <= 1: exp, the row sum
+    # and the product with its reciprocal are each off by a few units in the
+    # last place, 8 together, and that of a p near 1 stays when 1 is taken off
+    assert np.max(np.abs(got - g)) <= 8 * 2.0 ** -23 / 9
+
+
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 def test_softmax_backward(dev, dt):
     D, K = _dev()
