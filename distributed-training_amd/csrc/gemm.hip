@@ -354,7 +354,7 @@ static void pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cu
 // and the small-product kernel 0.45 (float64 0.55): it re-reads its operands for
 // every 32 x 32 tile through the L1. A split adds a launch and its partials'
 // traffic (about 6 TB/s from the last-level cache); where the next pass takes the
-// partials (`fused`: LayerNorm forward or backward, the row dots), only the
+// partials (`fused`: as LayerNorm or the row dots do), only the
 // partials beyond the output itself. Measured, 128 -> chosen:
 // [512, 512] x [512, 128] 23.9 -> 6.0 us (small-product), [1000, 256] x [256, 768]
 // float64 44.6 -> 14 us (small-product), [1500, 384] x [384, 1000] 34 -> 18 us (64),
@@ -378,10 +378,13 @@ static int64_t k_of_splits(int64_t K, int splits) {
   return kps < kBKT<T> ? kBKT<T> : kps;
 }
 
-// GemmArgs::fold_groups of an unsplit or thinly split range: about every 480 k
-// (a group is the 64 x 64 tile's 6 stages)
+// GemmArgs::fold_groups of an unsplit or thinly split range: every 192 k (a
+// group is the 64 x 64 tile's 6 stages). The 128-wide plan would have split k
+// over several blocks; at every 480 k the weight gradients of a block at 16 x
+// 114 x 576 were further from float64 than with that plan (5.5e-7, 4.6e-7), at
+// 192 they are nearer (3.9e-7), in the same time.
 template <typename T>
-constexpr int kFoldGroups = sizeof(T) == 4 ? 5 : 10;
+constexpr int kFoldGroups = sizeof(T) == 4 ? 2 : 4;
 
 // The small-product kernel with kps of k per wave: its loads' rate, or the chain
 // of one wave's MFMAs (which start behind its first loads).
@@ -445,7 +448,10 @@ static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const vo
   int64_t kps = k_of_splits<T>(K, splits);
   if (dma && !x6 && force_splits <= 0 && K > 0) {
     // 7 % below the 128-wide plan's estimate before leaving it
-    const bool fused = ep.ln_out || ep.parts_out || ep.rowdot_out;
+    // the shape alone decides, so that a product gives the same bits whether or
+    // not the next pass takes its partials: from one 128-wide tile per CU on,
+    // the other kernels have to beat that plan with its partials taken
+    const bool fused = tmn * batch >= cus;
     double best = 0.93 * tile_cost(M, N, K, batch, cus, bm, bn, splits, sizeof(T), fused);
     const int64_t t32 = cdiv(M, 32) * cdiv(N, 32) * batch;
     // Float32 products with a dimension of at most 256 (every product of a small
