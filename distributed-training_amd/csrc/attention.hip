@@ -1793,12 +1793,19 @@ static int attn_bwd_wide(AttnArgs& a) {
 // lane's Q slice (its query c, d = 16 g .. 16 g + 15, times scale * log2(e))
 // in registers; P feeds O^T += V^T P^T from registers; the next key tile's K
 // and V rows are prefetched into registers while the current one is computed.
-// Lazy rescaling against a reference max as in attn_fwd_kernel. With W > 1 the
-// waves take the key tiles in turn, each against a reference of its own, and
-// join their sums through LDS at the end of a query tile: a few heads of a long
-// sequence are too few pairs to fill the chip with one wave each, and the
-// chain of dependent MFMAs per query is W times shorter. At DP = 128 a wave
-// needs 220 to 256 registers, two per SIMD.
+// Lazy rescaling against a reference max as in attn_fwd_kernel; it starts at the
+// lowest finite number, so that scores of -inf add 2^(-inf) = 0 also where a
+// wave has seen no other yet (against -inf they would add NaN: the first tile of
+// wave w is key tile w, of which query 16 w sees one key). A query with no
+// finite score is left as the kernels that take unaligned operands of its head
+// dimension leave it: 0 with sum 0 (D up to 64), NaN (above); NaN in the aligned
+// form. With W > 1 the waves take the key tiles in turn, each against a
+// reference of its own, and join their sums through LDS at the end of a query
+// tile: a few heads of a long sequence are too few pairs to fill the chip with
+// one wave each, and the chain of dependent MFMAs per query is W times shorter.
+// At DP = 128 a wave needs 220 to 256 registers, two per SIMD.
+constexpr float kLowest = -3.40282347e38f;  // the lowest finite float
+
 template <int DP, int W, bool RAG>
 __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(AttnArgs a) {
   using M = A16<float>;
@@ -1880,7 +1887,7 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
     AT o[N];
 #pragma unroll
     for (int t = 0; t < N; ++t) o[t] = AT(0);
-    float mref = -INFINITY, mtop = -INFINITY, l = 0.f;
+    float mref = kLowest, mtop = -INFINITY, l = 0.f;
     fetch(wave);
     put();
     drain_vm();
@@ -1909,7 +1916,7 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
       mtop = fmaxf(mtop, bmax);
       if (__any(bmax > mref + kLazyLog2)) {
         const float mnew = fmaxf(mref, gmax(bmax));
-        const float alpha = ex2(mref - mnew);  // mref = -inf on the first tile: 0
+        const float alpha = ex2(mref - mnew);  // mref lowest on the first tile: 0
         l *= alpha;
 #pragma unroll
         for (int t = 0; t < N; ++t) o[t] *= alpha;
@@ -1937,7 +1944,7 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
     mtop = gmax(mtop);
     if constexpr (W > 1) {
       // the waves' outputs and sums against the largest of their reference
-      // maxima (a wave without a key tile: -inf, weight 0), added in wave
+      // maxima (a wave without a key tile has sums of 0), added in wave
       // order; wave w finishes registers w, w + W, ...
 #pragma unroll
       for (int t = 0; t < N; ++t)
@@ -1974,7 +1981,8 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
         }
       __syncthreads();  // read before the next segment's tiles overwrite them
     }
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    constexpr float kNone = RAG && DP == 64 ? 0.f : NAN;
+    const float inv = l > 0.f ? 1.f / l : kNone;
     // lane (g, c) register i of tile t: d = N (4 g + i) + t of query c
     if (!RAG || q0 + c < Tn) {
       float* orow = O + (int64_t)(q0 + c) * a.so.t;
@@ -1987,7 +1995,7 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
       }
       if (g == 0 && wave == 0) {
         ((float*)a.rowmax)[(int64_t)bh * Tn + q0 + c] = mtop;
-        ((float*)a.rowsum)[(int64_t)bh * Tn + q0 + c] = l * ex2(mref - mtop);
+        ((float*)a.rowsum)[(int64_t)bh * Tn + q0 + c] = l == 0.f ? kNone : l * ex2(mref - mtop);
       }
     }
     wave_sync();  // the last tile's rows are read before the next segment's put

@@ -351,3 +351,36 @@ def test_paired_ranges_at_ragged_lengths_and_other_head_dimensions(dev, T, D_):
         else:
             assert rel_err(gd[:T, :1, i].transpose(1, 2, 0, 3), ref) <= tol
     assert np.all(go[T:] == 7.0) and np.all(gd[T:] == 7.0)
+
+
+@pytest.mark.parametrize("T,D_", [(100, 36), (100, 64), (96, 64), (100, 80), (100, 96), (100, 128)])
+def test_scores_of_minus_infinity(dev, T, D_):
+    """Scores that overflow to -inf have probability 0, wherever they lie: the
+    first keys that a query sees, the whole of a 16-key tile, or the one key
+    that is unmasked in the first tile of one of a block's waves (key 16 w
+    for query 16 w). A product q[i, d] k[j, d] of -9e40 in one of the first
+    four dimensions makes them; in the oracle's float64 the score is finite
+    and its probability 0 all the same. dQ and dK have entries of up to 3e20
+    in those four dimensions, so each dimension is held against its own
+    largest entry."""
+    D, K = _dev()
+    rng = np.random.default_rng(T + D_)
+    q, k, v, g = (rng.standard_normal((1, 2, T, D_)).astype(np.float32) for _ in range(4))
+    pairs = [((16,), (16,)), ((32,), (32,)), ((48,), (48,)), ((90, 91, 95), range(48))]
+    q[..., :4] = k[..., :4] = 0
+    for d, (qs, ks) in enumerate(pairs):
+        q[:, :, list(qs), d] = 3e20
+        k[:, :, list(ks), d] = -3e20
+    o_ref, p, scale = ops.attention_fwd(q, k, v)
+    refs = ops.attention_bwd(g, q, k, v, p, scale)
+    m_ref, l_ref = ops.row_stats(q, k)
+    dq_, dk_, dv_ = D.from_numpy(q), D.from_numpy(k), D.from_numpy(v)
+    o, rmax, rsum = K.attn_fwd(dq_, dk_, dv_)
+    tol = TOL[np.float32]
+    assert rel_err(o.numpy(), o_ref) <= tol
+    assert rel_err(rmax.numpy(), m_ref * np.log2(np.e)) <= tol
+    assert rel_err(rsum.numpy(), l_ref) <= tol
+    for got, ref in zip(K.attn_bwd(dq_, dk_, dv_, o, D.from_numpy(g), rmax, rsum), refs):
+        for d in range(4):
+            assert rel_err(got.numpy()[..., d], ref[..., d]) <= tol
+        assert rel_err(got.numpy()[..., 4:], ref[..., 4:]) <= tol
