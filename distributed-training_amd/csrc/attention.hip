@@ -98,6 +98,7 @@ struct AttnArgs {
   int64_t B, H, T, D;
   double scale;
   int vec;   // 16-byte global access allowed for every operand
+  int head_group;  // (batch, head)s per group of the ragged forward's block order (D up to 64)
   int ovec;  // the results (out, or dq, dk and dv) too, with D a multiple of the vector
 };
 
@@ -1821,7 +1822,17 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
   float* Ks = lds + wave * 2 * TILE;
   float* Vs = Ks + TILE;
   __shared__ float tops[W][MT];  // W > 1: the waves' true maxima per query
-  const int bh = blockIdx.x;
+  int bh = (int)blockIdx.x, p0 = (int)blockIdx.y;
+  if constexpr (RAG && DP == 64) {
+    // XCD x (blocks are dealt to the XCDs in turn) takes the x-th eighth of the
+    // blocks ordered by group of head_group (batch, head)s, then pair
+    const unsigned gy = gridDim.y, n = gridDim.x * gy, id = blockIdx.y * gridDim.x + blockIdx.x, xcd = id & 7;
+    const unsigned at = xcd * (n >> 3) + (xcd < (n & 7) ? xcd : (n & 7)) + (id >> 3);
+    const unsigned G = (unsigned)a.head_group, grp = at / (G * gy), r = at - grp * (G * gy);
+    const unsigned left = gridDim.x - grp * G, gn = left < G ? left : G;
+    p0 = (int)(r / gn);
+    bh = (int)(grp * G + r % gn);
+  }
   const int64_t b = bh / a.H, h = bh % a.H;
   const int Tn = (int)a.T, D = (int)a.D;
   const int nt = RAG ? 2 * ((Tn + 2 * MT - 1) / (2 * MT)) : Tn / MT;
@@ -1868,9 +1879,9 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
     x = fmaxf(x, __shfl_xor(x, 16, 64));
     return fmaxf(x, __shfl_xor(x, 32, 64));
   };
-  // pairs p = blockIdx.y, + gridDim.y, ...: more than one when the grid would
+  // pairs p0, p0 + gridDim.y, ...: more than one when the grid would
   // otherwise run in several rounds of resident blocks
-  for (int p = (int)blockIdx.y; p < nt / 2; p += (int)gridDim.y)
+  for (int p = p0; p < nt / 2; p += (int)gridDim.y)
   for (int seg = 0; seg < 2; ++seg) {
     const int qt = seg == 0 ? p : nt - 1 - p;
     const int q0 = qt * MT;
@@ -2064,7 +2075,23 @@ template <int DP, int W, bool RAG>
 static int attn_fwd_paired(AttnArgs& a) {
   static const int resident = resident_blocks(attn_fwd_p16_kernel<DP, W, RAG>, 64 * W);
   const unsigned pairs = (unsigned)cdiv(a.T, 32);
-  const unsigned per = pairs_per_block(a.B * a.H, pairs, resident);
+  unsigned per = pairs_per_block(a.B * a.H, pairs, resident);
+  if constexpr (RAG && DP == 64) {
+    // Every pair's block reads its head's K and V up to the pair's tiles: dealt
+    // pair by pair over all heads, the blocks that run together read more heads
+    // than an XCD's 4 MB L2 holds, and where B H is no multiple of 8 every XCD
+    // reads every head (the 128-row blocks of attn_fwd_kernel, a quarter of the
+    // reads, were faster). So an XCD takes its own heads, from 8 MB of K and V on in
+    // groups of up to 4 MB. From three rounds of blocks on, one pair per
+    // block: rounds at full occupancy beat fewer blocks of several pairs. At D 64,
+    // before, with both, attn_fwd_kernel: B H 442, T 499 279, 190, 198 us; 126, 1500
+    // 584, 420, 424 us; 1024, 333 277, 217, 273 us; 512, 615 378, 320, 340 us; 64,
+    // 499 32, 32, 52 us.
+    const int64_t share = cdiv(a.B * a.H, 8), bytes = share * a.T * a.D * 8;
+    const int64_t groups = bytes > ((int64_t)8 << 20) ? cdiv(bytes, (int64_t)4 << 20) : 1;
+    a.head_group = (int)cdiv(share, groups);
+    if (a.B * a.H * (int64_t)pairs > 2 * (int64_t)resident * num_cus()) per = 1;
+  }
   attn_fwd_p16_kernel<DP, W, RAG><<<dim3((unsigned)(a.B * a.H), (unsigned)cdiv(pairs, per)), 64 * W, 0, stream()>>>(a);
   LAUNCH_CHECK("attn_fwd_p16_kernel");
   return DTMI_OK;

@@ -110,21 +110,27 @@ def test_backward_paired_ranges_at_every_pair_count(dev, T):
             assert bits_equal(x, y)
 
 
-@pytest.mark.parametrize("B,H,T", [(40, 8, 256), (36, 4, 352), (40, 8, 512)])
-def test_paired_grid_shapes_agree_bit_for_bit(dev, B, H, T):
+@pytest.mark.parametrize("B,H,T,D_", [(40, 8, 256, 64), (36, 4, 352, 64), (40, 8, 512, 64), (40, 8, 345, 64),
+                                      (33, 13, 345, 64), (64, 8, 345, 64), (33, 13, 345, 48), (40, 8, 345, 96),
+                                      (40, 8, 345, 128)])
+def test_paired_grid_shapes_agree_bit_for_bit(dev, B, H, T, D_):
     """The float32 paired-range passes pick their grids by size: the dQ pass
     takes four query-tile pairs per block when there are at least two such
     blocks per CU, else two pairs with each query tile's d-tiles split over two
     waves; the key pass and the forward take several tile pairs per block when
     one pair per block would need more than one round of resident blocks (at
     T 352 the key pass's 11 pairs do not divide evenly over the blocks; at
-    T 512 the forward takes two pairs per block). Each order of additions is
-    the same either way, so a (batch, head) gets the same bits: the full batch
-    against its first two batch elements alone (split d-tiles, one pair per
-    block), and those against the oracle."""
+    T 512 the forward takes two pairs per block). At lengths that are no
+    multiple of 32 the forward up to D = 64 also deals its blocks in another
+    order, whole heads to an XCD (429 heads: not a multiple of 8; 512 heads at
+    T 345: several groups per XCD), and above it the key pass's and the
+    forward's four waves reuse their LDS from pair to pair. Each order of
+    additions is the same either way, so a (batch, head) gets the same bits:
+    the full batch against its first two batch elements alone (split d-tiles,
+    one pair per block), and those against the oracle."""
     D, K = _dev()
     rng = np.random.default_rng(B + T)
-    q, k, v, g = (rng.standard_normal((B, H, T, 64)).astype(np.float32) for _ in range(4))
+    q, k, v, g = (rng.standard_normal((B, H, T, D_)).astype(np.float32) for _ in range(4))
 
     def bwd(sl):
         x = [D.from_numpy(np.ascontiguousarray(t[sl])) for t in (q, k, v, g)]
