@@ -8,6 +8,7 @@
 // The big-array kernels (GELU, binary same-shape, column sums) are HBM-bound:
 // 16-byte vector access when aligned, grid-stride loops, no atomics.
 #include <cmath>
+#include <cstdint>
 
 #include "colreduce.h"
 #include "common.h"
@@ -582,13 +583,29 @@ DTMI_EXPORT int dtmi_reduce_sum(int dtype, void* out, const void* x, const int64
     LAUNCH_CHECK("reduce_lead_kernel");
     return DTMI_OK;
   }
-  // A group of lanes per output when the innermost axis is reduced (the terms
-  // of one output are neighbours) or there is one output, from 32 terms on:
-  // below that, and where the outputs are the neighbours, a thread per output
-  // reads whole lines and needs no combining.
+  // A group of lanes per output when the innermost axis is reduced or there is
+  // one output, from 32 terms on, unless a thread per output does it faster. By
+  // the smaller stride, the terms of one output are neighbours, or (a transposed
+  // view) consecutive outputs are. Outputs that are neighbours are read line by
+  // line by their threads, bound by one thread's chain of loads until there are
+  // enough threads: 65536 x 32 16 us (17 with groups), 65536 x 64 29 (24), 131072 x
+  // 64 37 (44), 262144 x 32 31 (60), 1048576 x 64 186 (441), 4096 x 512 210 (17).
+  // Neighbouring terms: groups, but for 32 to 35 terms (half of a wave is idle) of
+  // outputs that fill the chip and whose rows the L1s still hold: 65536 x 32 17 us
+  // (15 with groups), 131072 x 32 22 (27), 262144 x 32 35 (55), 262144 x 40 70
+  // (55), 524288 x 32 270 (107).
   int inner = ndim - 1;
   while (inner > 0 && shape[inner] == 1) --inner;
-  if (nred >= 32 && nout <= (1LL << 23) && (nout == 1 || (inner >= 0 && reduce_mask[inner]))) {
+  int64_t s_red = INT64_MAX, s_kept = 0;  // smallest reduced stride; the innermost kept axis's
+  for (int k = 0; k < ndim; ++k) {
+    const int64_t st = strides ? strides[k] : cstr[k], m = st < 0 ? -st : st;
+    if (shape[k] == 1 || m == 0) continue;
+    if (!reduce_mask[k]) s_kept = m;
+    else if (m < s_red) s_red = m;
+  }
+  const bool by_thread = s_kept > 0 && s_kept < s_red ? nout >= 131072 || (nout >= 65536 && nred < 48)
+                                                      : nred < 36 && nout >= 98304 && nout <= 262144;
+  if (nred >= 32 && nout <= (1LL << 23) && !by_thread && (nout == 1 || (inner >= 0 && reduce_mask[inner]))) {
     // one stride over all reduced axes, when each outer one continues the inner
     int64_t rs = 0, span = 1;
     for (int k = ndim - 1; k >= 0; --k) {

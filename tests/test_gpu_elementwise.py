@@ -117,3 +117,20 @@ def test_sums_over_trailing_axes(dev, dt, shape, axes):
     if len(shape) == 2:  # a strided view of the same numbers
         t = K.reduce_sum(D.from_numpy(np.ascontiguousarray(x.T)).transpose(1, 0), axes).numpy()
         assert np.all(np.abs(t - ref) <= bound)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("shape,perm", [((32, 100003), (1, 0)), ((64, 131072), (1, 0)), ((100, 200001), (1, 0)),
+                                        ((50, 2000, 256), (2, 1, 0)), ((500, 40, 300), (0, 2, 1)),
+                                        ((150000, 33), (0, 1))])
+def test_sums_of_many_outputs_over_a_views_last_axis(dev, dt, shape, perm):
+    """Views with more than 65536 outputs that are neighbours in memory (a
+    transposed view's last axis), or with 32 to 39 terms each: one thread per
+    output adds its terms in order, so the bits are those of an explicit sum."""
+    D, K = _dev()
+    x = np.random.default_rng(sum(shape)).standard_normal(shape).astype(dt)
+    v = x.transpose(perm)
+    ref = np.zeros(v.shape[:-1], dt)
+    for r in range(v.shape[-1]):
+        ref = ref + v[..., r]
+    assert bits_equal(K.reduce_sum(D.from_numpy(x).transpose(*perm), [v.ndim - 1]).numpy(), ref)
