@@ -254,8 +254,6 @@ __global__ void __launch_bounds__(1024) xent_fused_kernel(float* __restrict__ dz
   }
 }
 
-constexpr int64_t kFusedRagged = 1024;  // see dtmi_xent_fused
-
 // x *= g[0] unless g[0] == 1 (then x is already the gradient).
 template <typename T>
 __global__ void __launch_bounds__(256) xent_grad_scale_kernel(T* __restrict__ x, const T* __restrict__ g, int64_t n) {
@@ -351,13 +349,15 @@ DTMI_EXPORT int dtmi_xent_fused(int dtype, void* loss, void* dlogits, void* rowm
              (long long)rows, (long long)vocab);
   DTMI_CHECK(loss && dlogits && rowmax && rowsum && logits && targets, "dtmi_xent_fused: NULL pointer");
   const int64_t nv = vocab / 4;
-  // A vocabulary that is no multiple of 4 takes the one-pass form above 1024
-  // logits: 2048 x 20001 119 -> 94 us, 2048 x 4099 31 -> 22, 1024 x 2049
-  // 19.7 -> 16.9, 2048 x 1027 level; below, a row leaves most of its block
-  // without a vector (4096 x 65 19 us with two kernels, 31 with one).
+  // A vocabulary that is no multiple of 4 takes the one-pass form where it is the
+  // faster: above 1024 logits up to 2048 rows (launches count), above 1750 for
+  // more. Shorter rows leave most of their 1024 threads without a vector. Two
+  // kernels and one: 64 x 1025 15 and 9 us, 1024 x 1501 17 and 14, 2048 x 1027
+  // level, 4096 x 1025 25.5 and 31, 16384 x 1501 97 and 111, 16384 x 1801 level,
+  // 8192 x 3001 79 and 61, 2048 x 20001 119 and 94, 4096 x 65 19 and 31.
   const bool rag = vocab % 4 != 0;
   const bool fused = dtype == DTMI_F32 && nv <= 16 * 1024 && aligned(logits, 16) && aligned(dlogits, 16) &&
-                     (!rag || vocab > kFusedRagged);
+                     (!rag || vocab > (rows <= 2048 ? 1024 : 1750));
   if (!fused) {  // the two-kernel form: forward, then the gradient for an upstream gradient of 1
     int rc = dtmi_xent_fwd(dtype, loss, rowmax, rowsum, logits, targets, rows, vocab);
     if (rc) return rc;

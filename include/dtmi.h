@@ -257,8 +257,9 @@ int dtmi_xent_bwd(int dtype, void* dlogits, const void* logits, const void* rowm
 /* Forward and gradient together, for a training step: the dtmi_xent_fwd outputs
  * plus dlogits for an upstream gradient of 1, i.e. (exp(z - max) / sum -
  * onehot(t)) / rows (dtrain/autograd.py:262-265 with g = 1). float32 rows of
- * up to 65536 logits are read once and dlogits written once; other shapes run
- * the two kernels above. dtmi_xent_grad_scale then multiplies dlogits (n
+ * up to 65536 logits are read once and dlogits written once (lengths that are
+ * no multiple of 4: from 1025 on, from 1751 on above 2048 rows); other shapes
+ * run the two kernels above. dtmi_xent_grad_scale then multiplies dlogits (n
  * elements) in place by the device scalar *g_dev unless it is exactly 1. */
 int dtmi_xent_fused(int dtype, void* loss, void* dlogits, void* rowmax, void* rowsum, const void* logits,
                     const int64_t* targets, int64_t rows, int64_t vocab);

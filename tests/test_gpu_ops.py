@@ -197,6 +197,26 @@ def test_cross_entropy_single_pass_with_rows_off_the_16_byte_grid(dev, V):
     assert np.max(np.abs(got - g)) <= 8 * 2.0 ** -23 / 9
 
 
+@pytest.mark.parametrize("rows,V,one_pass", [(2048, 1025, True), (2049, 1025, False), (2049, 1749, False),
+                                             (2049, 1751, True)])
+def test_cross_entropy_form_by_rows_and_vocabulary(dev, rows, V, one_pass):
+    """Either side of the lines between the one-pass form and the two kernels
+    (whose bits the forward and backward entry points give), against the
+    oracle."""
+    D, K = _dev()
+    rng = np.random.default_rng(rows + V)
+    z = (rng.standard_normal((rows, V)) * 3).astype(np.float32)
+    t = rng.integers(0, V, rows)
+    loss, cache = ops.cross_entropy_fwd(z, t)
+    g = ops.cross_entropy_bwd(np.asarray(1.0, dtype=np.float32), z, t, cache)
+    dz, dt_ = D.from_numpy(z), D.from_numpy(t.astype(np.int64))
+    dloss, _, _, dl = K.xent_fused(dz, dt_)
+    assert rel_err(dloss.numpy(), loss) <= TOL[np.float32]
+    assert rel_err(dl.numpy(), g) <= TOL[np.float32]
+    _, rmax, rsum = K.xent_fwd(dz, dt_)
+    assert bits_equal(dl.numpy(), K.xent_bwd(dz, dt_, rmax, rsum).numpy()) != one_pass
+
+
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 def test_softmax_backward(dev, dt):
     D, K = _dev()
