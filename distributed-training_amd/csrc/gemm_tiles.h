@@ -83,9 +83,19 @@ __device__ __forceinline__ void init_ptr(TilePtr<T, KCONTIG, BMN>& t, const T* _
   }
 }
 
+// A k-tile wholly in range; the pointers advance by `step` elements to the next.
+template <typename T, bool KCONTIG, int BMN>
+__device__ __forceinline__ void load_full(TileRegs<T, KCONTIG, BMN>& r, TilePtr<T, KCONTIG, BMN>& t, int64_t step) {
+#pragma unroll
+  for (int i = 0; i < TileLayout<T, KCONTIG, BMN>::NVEC; ++i) {
+    r.v[i] = *reinterpret_cast<const typename MF<T>::vec_t*>(t.p[i]);
+    t.p[i] += step;
+  }
+}
+
 // The last k-tile when it extends past kend: the same number of loads as a
 // full tile, from addresses clamped into [kbeg, kend) (k past kend is zeroed
-// when the tile is stored to LDS, see dma_tail_store).
+// when the tile is stored to LDS, see store_tile and dma_tail_store).
 template <typename T, bool KCONTIG, int BMN>
 __device__ __forceinline__ void load_tail(TileRegs<T, KCONTIG, BMN>& r, const TilePtr<T, KCONTIG, BMN>& t,
                                           int64_t ld, int64_t k0, int64_t kend) {
@@ -107,20 +117,19 @@ __device__ __forceinline__ void load_tail(TileRegs<T, KCONTIG, BMN>& r, const Ti
   }
 }
 
-template <typename T, bool KCONTIG, int BMN>
-__device__ __forceinline__ void store_tile(T* __restrict__ lds, const TileRegs<T, KCONTIG, BMN>& r) {
+// Registers -> LDS; TAIL: vectors whose k is `left` or more past the tile's first as zeros.
+template <bool TAIL, typename T, bool KCONTIG, int BMN>
+__device__ __forceinline__ void store_tile(T* __restrict__ lds, const TileRegs<T, KCONTIG, BMN>& r, int left) {
   using L = TileLayout<T, KCONTIG, BMN>;
   constexpr int VEC = L::VEC;
   constexpr int kBK = L::kBK;
 #pragma unroll
   for (int i = 0; i < L::NVEC; ++i) {
     const int f = threadIdx.x + 256 * i;
-    int off;
-    if (KCONTIG)
-      off = (f / (kBK / VEC)) * L::STRIDE + (f % (kBK / VEC)) * VEC;
-    else
-      off = (f / (BMN / VEC)) * L::STRIDE + (f % (BMN / VEC)) * VEC;
-    *reinterpret_cast<typename MF<T>::vec_t*>(lds + off) = r.v[i];
+    const int row = KCONTIG ? f / (kBK / VEC) : f / (BMN / VEC);
+    const int col = (KCONTIG ? f % (kBK / VEC) : f % (BMN / VEC)) * VEC;
+    const bool in = !TAIL || (KCONTIG ? col : row) < left;
+    *reinterpret_cast<typename MF<T>::vec_t*>(lds + row * L::STRIDE + col) = in ? r.v[i] : typename MF<T>::vec_t(0);
   }
 }
 
@@ -240,9 +249,12 @@ __device__ __forceinline__ void write_acc(const GemmArgs& a, const typename MF<T
 }
 
 // Leading dimensions beyond the 32-bit offsets of gemm_dma_kernel: registers ->
-// LDS, element loads, any alignment. Block tile BM x BN, 4 waves in a 2 x 2 grid
-// of (BM/2) x (BN/2) wave tiles.
-template <typename T, int BM, int BN, bool AKC, bool BKC>
+// LDS. VECA / VECB: a 16-byte granular operand is read as vectors through
+// per-thread pointers advanced by a k-tile (float32 [256, 4096] x [4096, 256],
+// rows of A 2^24 bytes apart: 36 us, 59 element by element); others element by
+// element. Block tile BM x BN, 4 waves in a 2 x 2 grid of (BM/2) x (BN/2) wave
+// tiles.
+template <typename T, int BM, int BN, bool AKC, bool BKC, bool VECA, bool VECB>
 __global__ void __launch_bounds__(256, 2) gemm_kernel(GemmArgs a) {
   constexpr int kBK = kBKT<T>;
   using MFT = MF<T>;
@@ -280,18 +292,39 @@ __global__ void __launch_bounds__(256, 2) gemm_kernel(GemmArgs a) {
   TileRegs<T, AKC, BM> ra;
   TileRegs<T, BKC, BN> rb;
   const int64_t ntiles = kend > kbeg ? (kend - kbeg + kBK - 1) / kBK : 0;
+  const int64_t nfull = kend > kbeg ? (kend - kbeg) / kBK : 0;
+  TilePtr<T, AKC, BM> pa;
+  TilePtr<T, BKC, BN> pb;
+  if (VECA) init_ptr<T, AKC, BM>(pa, A, a.lda, m0, a.M, kbeg);
+  if (VECB) init_ptr<T, BKC, BN>(pb, B, a.ldb, n0, a.N, kbeg);
+  // Tiles are loaded in order kt = 0, 1, ...; only the last can be partial.
   auto load = [&](int64_t kt) {
     const int64_t k0 = kbeg + kt * kBK;
-    load_tile<T, AKC, BM>(ra, A, a.lda, m0, a.M, k0, kend);
-    load_tile<T, BKC, BN>(rb, B, a.ldb, n0, a.N, k0, kend);
+    if (kt < nfull) {
+      if (VECA) load_full<T, AKC, BM>(ra, pa, AKC ? (int64_t)kBK : kBK * a.lda);
+      if (VECB) load_full<T, BKC, BN>(rb, pb, BKC ? (int64_t)kBK : kBK * a.ldb);
+    } else {
+      if (VECA) load_tail<T, AKC, BM>(ra, pa, a.lda, k0, kend);
+      if (VECB) load_tail<T, BKC, BN>(rb, pb, a.ldb, k0, kend);
+    }
+    if (!VECA) load_tile<T, AKC, BM>(ra, A, a.lda, m0, a.M, k0, kend);
+    if (!VECB) load_tile<T, BKC, BN>(rb, B, a.ldb, n0, a.N, k0, kend);
   };
-  auto store = [&](int stage) {
-    store_tile<T, AKC, BM>(lds + stage * LA::SIZE, ra);
-    store_tile<T, BKC, BN>(lds + 2 * LA::SIZE + stage * LB::SIZE, rb);
+  auto store = [&](int64_t kt, int stage) {
+    T* As = lds + stage * LA::SIZE;
+    T* Bs = lds + 2 * LA::SIZE + stage * LB::SIZE;
+    if (kt < nfull) {
+      store_tile<false, T, AKC, BM>(As, ra, 0);
+      store_tile<false, T, BKC, BN>(Bs, rb, 0);
+    } else {
+      const int left = (int)(kend - kbeg - kt * kBK);
+      store_tile<true, T, AKC, BM>(As, ra, left);
+      store_tile<true, T, BKC, BN>(Bs, rb, left);
+    }
   };
   if (ntiles > 0) {
     load(0);
-    store(0);
+    store(0, 0);
   }
   __syncthreads();
   const bool take_colsum = a.colsum != nullptr && tm == 0 && (int)threadIdx.x < BN;
@@ -323,7 +356,7 @@ __global__ void __launch_bounds__(256, 2) gemm_kernel(GemmArgs a) {
       for (int k = 0; k < kBK; ++k) t = t + (BKC ? Bs[threadIdx.x * LB::STRIDE + k] : Bs[k * LB::STRIDE + threadIdx.x]);
       csum += (double)t;
     }
-    if (kt + 1 < ntiles) store(cur ^ 1);
+    if (kt + 1 < ntiles) store(kt + 1, cur ^ 1);
     __syncthreads();
   }
   if (take_colsum) finish_colsum<T>(a, csum, n0 + threadIdx.x, split);
@@ -703,8 +736,16 @@ __global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(
 template <typename T, int BM, int BN, bool AKC, bool BKC>
 static void launch_variant(const GemmArgs& a, dim3 grid, bool veca, bool vecb, bool dma) {
   if (!dma) {
-    if constexpr (BM == 128 && BN == 128)  // the other tiles: gemm_dma_kernel only (see gemm_impl)
-      gemm_kernel<T, BM, BN, AKC, BKC><<<grid, 256, 0, stream()>>>(a);
+    if constexpr (BM == 128 && BN == 128) {  // the other tiles: gemm_dma_kernel only (see gemm_impl)
+      if (veca && vecb)
+        gemm_kernel<T, BM, BN, AKC, BKC, true, true><<<grid, 256, 0, stream()>>>(a);
+      else if (veca)
+        gemm_kernel<T, BM, BN, AKC, BKC, true, false><<<grid, 256, 0, stream()>>>(a);
+      else if (vecb)
+        gemm_kernel<T, BM, BN, AKC, BKC, false, true><<<grid, 256, 0, stream()>>>(a);
+      else
+        gemm_kernel<T, BM, BN, AKC, BKC, false, false><<<grid, 256, 0, stream()>>>(a);
+    }
   } else if (veca && vecb) {
     gemm_dma_kernel<T, BM, BN, AKC, BKC, true, true><<<grid, 256, 0, stream()>>>(a);
   } else if (veca) {

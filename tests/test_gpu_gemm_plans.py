@@ -72,3 +72,51 @@ def test_linear_backward_column_sums_and_epilogues(dev, dt, M, K, N):
     assert np.all(np.abs(y.numpy() - (X @ W + b + r)) <= bound)
     h, act = K_.linear_fwd_fused(D.from_numpy(x), D.from_numpy(w), D.from_numpy(b), gelu=True)
     assert bits_equal(act.numpy(), K_.gelu_fwd(h).numpy())
+
+
+def _strided(a, ld):
+    """`a` in HBM with rows `ld` elements apart, NaN between them."""
+    from dtmi import device as D
+    buf = D.full(((a.shape[0] - 1) * ld + a.shape[1],), np.nan, a.dtype)
+    v = D.DeviceArray(buf.block, a.shape, a.dtype, 0, (ld, 1))
+    v.assign(a)
+    return v
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+@pytest.mark.parametrize("pad_a,pad_b", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_leading_dimensions_of_2_24_bytes(dev, dt, akc, bkc, pad_a, pad_b):
+    """Leading dimensions beyond the direct-to-LDS kernel's 32-bit offsets take the
+    register-staged kernel: 16-byte granular operands as vectors, others element
+    by element, with ragged M and N, a partial last k-tile and a split of k.
+    Small whole numbers, so that every order of the sums gives the exact result."""
+    from dtmi import _lib, device as D
+    M, N, K = 132, 68, 76
+    rng = np.random.default_rng(M + pad_a + 2 * pad_b)
+    A = rng.integers(-8, 9, (M, K) if akc else (K, M)).astype(dt)
+    B = rng.integers(-8, 9, (N, K) if bkc else (K, N)).astype(dt)
+    bias = rng.integers(-8, 9, N).astype(dt)
+    ld = (1 << 24) // np.dtype(dt).itemsize
+    da, db, dbias = _strided(A, ld + pad_a), _strided(B, ld + pad_b), D.from_numpy(bias)
+    ref = (A if akc else A.T) @ (B.T if bkc else B) + bias
+    for splits in (0, 1, 2):
+        C = D.full((M, N), 7.0, dt)
+        _lib.call("dtmi_gemm", _lib.dtype_code(dt), int(akc), int(bkc), M, N, K, da.ptr, ld + pad_a, 0, db.ptr,
+                  ld + pad_b, 0, C.ptr, N, 0, 1, dbias.ptr, 0, splits)
+        assert np.array_equal(C.numpy(), ref)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_weight_gradient_and_column_sums_of_rows_of_2_24_bytes(dev, dt, pad):
+    """dW and db where a row of dY is 2^24 bytes: the register-staged kernel's
+    column sums, exact on small whole numbers."""
+    from dtmi import _lib, device as D
+    M, K, N = 37, 4, (1 << 24) // np.dtype(dt).itemsize + pad
+    rng = np.random.default_rng(N)
+    x, g = (rng.integers(-8, 9, s, dtype=np.int8).astype(dt) for s in ((M, K), (M, N)))
+    dx, dg, dw, db = D.from_numpy(x), D.from_numpy(g), D.empty((K, N), dt), D.empty((N,), dt)
+    _lib.call("dtmi_linear_bwd_dw", _lib.dtype_code(dt), dw.ptr, db.ptr, dx.ptr, dg.ptr, M, K, N, 0)
+    assert np.array_equal(dw.numpy(), x.T @ g)
+    assert np.array_equal(db.numpy(), g.sum(axis=0))
