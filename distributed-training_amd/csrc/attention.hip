@@ -2145,8 +2145,8 @@ static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
   int form = paired_form<T>(a, true);
   // dS for the dQ pass: B*H*T*T elements (the causal tiles only on the
   // paired-range path), up to g_max_ds_bytes; beyond that the dQ pass
-  // recomputes S, P and dP itself, or (D above 64) the scores of one batch
-  // element are materialised.
+  // recomputes S, P and dP itself, or (D above 64, also where the memory for dS
+  // is not to be had) the scores of one batch element are materialised.
   a.ds = nullptr;
   const double ds_bytes = form ? (double)a.B * a.H * (double)ds16_tiles(2 * cdiv(a.T, 32)) * 256.0 * sizeof(T)
                                : (double)a.B * a.H * a.T * a.T * sizeof(T);
@@ -2162,7 +2162,8 @@ static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
     rc = pool_alloc(&a.ds, (size_t)ds_bytes);
     if (rc) {
       pool_free(drow);
-      return rc;
+      // materialised scores need two [H, T, T] arrays, whatever the batch
+      return dp < 0 && rc == DTMI_ERR_OOM ? attn_bwd_wide<T>(a) : rc;
     }
   }
   {

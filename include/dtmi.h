@@ -376,9 +376,10 @@ int dtmi_linear_bwd_dx_parts(int dtype, void* parts, int max_parts, int* nparts,
 
 /* ------------------------------------------------------- causal attention
  * dtrain/autograd.py:226-247: o = softmax(q k^T * scale + causal mask) v over
- * (B, H, T, D), the head dimension D contiguous (up to 64 in the fused MFMA
- * kernels; above 64 through materialised scores and batched GEMMs, one batch
- * element at a time); each *_strides argument points at three
+ * (B, H, T, D), the head dimension D contiguous (up to 64, and float32 up to
+ * 128 with 16-byte aligned rows, in the fused MFMA kernels; others through
+ * materialised scores and batched GEMMs, one batch element at a time); each
+ * *_strides argument points at three
  * element strides (b, h, t) of that operand, so q/k/v/o/dq/dk/dv may be views
  * into fused [B, T, 3, H, D] / [B, T, H, D] buffers. The forward writes o and
  * the per-row softmax statistics (contiguous [B, H, T]): rowmax = log2(e) *
@@ -404,10 +405,13 @@ int dtmi_attn_bwd_rowsum(int dtype, int64_t B, int64_t H, int64_t T, int64_t D, 
                          void* dq, const int64_t* dq_strides, void* dk, const int64_t* dk_strides, void* dv,
                          const int64_t* dv_strides);
 /* The backward's dQ pass reads the dS = P * (dP - rowsum(dO * O)) that its key
- * pass wrote to a pooled [B, H, T, T] workspace when that takes at most
- * `bytes` (default 4 GiB), and otherwise recomputes S, P and dP itself (the
- * same products as dtrain/autograd.py:239-246). Sets the bound (0: always
- * recompute) and returns the previous one in *previous (if not NULL). */
+ * pass wrote to a pooled [B, H, T, T] workspace (float32 with D of 36 to 128 and
+ * 16-byte aligned rows: its causal half) when that takes at most `bytes`
+ * (default 4 GiB), and otherwise recomputes S, P and dP itself (the same
+ * products as dtrain/autograd.py:239-246). Above D = 64 the other way is
+ * materialised scores, two pooled [H, T, T] arrays; float32 takes it also where
+ * the workspace cannot be allocated. Sets the bound (0: always recompute) and
+ * returns the previous one in *previous (if not NULL). */
 int dtmi_attn_set_ds_limit(int64_t bytes, int64_t* previous);
 
 #ifdef __cplusplus

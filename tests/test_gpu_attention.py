@@ -236,6 +236,36 @@ def test_backward_without_the_ds_workspace_matches_with_it(dev):
         assert rel_err(full.numpy(), ref) <= 1e-5
 
 
+def test_wide_heads_without_memory_for_the_ds_workspace(dev):
+    """D above 64 where dS of the whole batch (576 batch elements of T 16384:
+    309 GB) cannot be allocated: the backward falls back to materialised scores,
+    two [H, T, T] arrays whatever the batch. The batch elements share their
+    inputs (stride 0), so each one's gradients are those of a batch of one by
+    the same route (bound 0), to the bit, and those of the dS route to the
+    float32 bar."""
+    D, K = _dev()
+    B, T, Dh = 576, 16384, 72
+    rng = np.random.default_rng(72)
+    q1, k1, v1, g1 = (D.from_numpy(rng.standard_normal((1, 1, T, Dh)).astype(np.float32)) for _ in range(4))
+    o1, m1, l1 = K.attn_fwd(q1, k1, v1)
+
+    def batch(x):
+        return D.DeviceArray(x.block, (B, 1, T, Dh), x.dtype, x.offset, (0, T * Dh, Dh, 1))
+    stats = [D.from_numpy(np.ascontiguousarray(np.broadcast_to(x.numpy(), (B, 1, T)))) for x in (m1, l1)]
+    by_ds = K.attn_bwd(q1, k1, v1, o1, g1, m1, l1)
+    prev = K.attn_set_ds_limit(1 << 50)
+    try:
+        got = K.attn_bwd(*(batch(x) for x in (q1, k1, v1, o1, g1)), *stats)
+        K.attn_set_ds_limit(0)
+        one = K.attn_bwd(q1, k1, v1, o1, g1, m1, l1)
+    finally:
+        K.attn_set_ds_limit(prev)
+    for x, r, d in zip(got, one, by_ds):
+        for b in (0, B - 1):
+            assert bits_equal(x[b].numpy(), r[0].numpy())
+        assert rel_err(r.numpy(), d.numpy()) <= TOL[np.float32]
+
+
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 @pytest.mark.parametrize("shape", [(2, 2, 64, 128), (1, 3, 100, 80), (2, 1, 33, 256)])
 def test_head_dimensions_beyond_64(dev, dt, shape):
