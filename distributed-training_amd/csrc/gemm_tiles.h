@@ -640,17 +640,18 @@ __global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(
   // One k-tile: this wave's loads of tile kt have landed (the NST - 2 tiles
   // after it may still be in flight), then every wave's have, and every wave is
   // done with the stage about to be refilled (that of tile kt - 1); then the
-  // loads of tile kt + NST - 1 and the MFMAs of tile kt.
+  // loads of tile kt + NST - 1 and the MFMAs of tile kt. The conditions have the
+  // form of the main loop's, so that those it implies fold away there (as
+  // nfull - 1 - kt >= ... each cost a branch a step: 8192 x 512 x 2048 130 -> 143 us).
   auto step = [&](auto stc, int kt) {
     constexpr int st = decltype(stc)::value;
-    const int after = nfull - 1 - kt;  // tiles issued or to be issued after kt
-    if (after >= NST - 2)
+    if (kt + NST - 2 < nfull)
       dma_wait_barrier<(NST - 2) * NQT>();
-    else if (NST > 5 && after == 3)
+    else if (NST > 5 && kt + 3 < nfull)
       dma_wait_barrier<(NST > 5 ? 3 : 0) * NQT>();
-    else if (NST > 4 && after == 2)
+    else if (NST > 4 && kt + 2 < nfull)
       dma_wait_barrier<(NST > 4 ? 2 : 0) * NQT>();
-    else if (NST > 3 && after == 1)
+    else if (NST > 3 && kt + 1 < nfull)
       dma_wait_barrier<(NST > 3 ? 1 : 0) * NQT>();
     else
       dma_wait_barrier<0>();
@@ -661,10 +662,18 @@ __global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(
     [&]<int... I>(std::integer_sequence<int, I...>) { (f(IC<I>()), ...); }(std::make_integer_sequence<int, NST>());
   };
   static_assert(NST >= 3 && NST <= 6 && (NST - 2) * NQT < 64, "waits of step(), vmcnt range");
-  each_stage([&](auto stc) {
-    constexpr int st = decltype(stc)::value;
-    if (st < NST - 1 && st < nfull) issue(stc);
-  });
+  // The three-stage kernels' steps are written out: run through each_stage they
+  // are the same instructions, but 8192 x 512 x 2048 took 146 us (137 written out)
+  // at the same cycle count, that is at a lower clock.
+  if constexpr (NST == 3) {
+    if (nfull > 0) issue(IC<0>());
+    if (nfull > 1) issue(IC<1>());
+  } else {
+    each_stage([&](auto stc) {
+      constexpr int st = decltype(stc)::value;
+      if (st < NST - 1 && st < nfull) issue(stc);
+    });
+  }
   // A long range without a K split is summed in pieces (a.fold_groups): a chain
   // of thousands of float32 additions would lose what the splits of the 128-wide
   // tiles keep. 32 vector instructions per 192 k beside 96 MFMAs, no difference
@@ -688,16 +697,27 @@ __global__ void __launch_bounds__(256, (BM + BN > 384 ? 1 : 2)) gemm_dma_kernel(
   };
   int kt = 0, grp = 0;
   for (; kt + NST <= nfull; kt += NST) {
-    each_stage([&](auto stc) { step(stc, kt + decltype(stc)::value); });
+    if constexpr (NST == 3) {
+      step(IC<0>(), kt);
+      step(IC<1>(), kt + 1);
+      step(IC<2>(), kt + 2);
+    } else {
+      each_stage([&](auto stc) { step(stc, kt + decltype(stc)::value); });
+    }
     if constexpr (FOLD)
       if (++grp == a.fold_groups) {
         fold();
         grp = 0;
       }
   }
-  each_stage([&](auto stc) {
-    if (kt + decltype(stc)::value < nfull) step(stc, kt + decltype(stc)::value);
-  });
+  if constexpr (NST == 3) {
+    if (kt < nfull) step(IC<0>(), kt);
+    if (kt + 1 < nfull) step(IC<1>(), kt + 1);
+  } else {
+    each_stage([&](auto stc) {
+      if (kt + decltype(stc)::value < nfull) step(stc, kt + decltype(stc)::value);
+    });
+  }
   const int st = nfull % NST;  // stage of the partial tile, if any
   if (ntiles > nfull) {  // the partial last k-tile, through registers
     const int64_t k0 = kbeg + (int64_t)nfull * BK;
