@@ -196,11 +196,13 @@ def test_attention_on_fused_qkv_layout(dev, dt):
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 @pytest.mark.parametrize("shape", [(1, 2, 4, 3), (2, 2, 5, 4), (2, 3, 100, 64), (1, 1, 257, 33), (16, 12, 256, 64),
-                                   (1, 2, 384, 64)])
+                                   (1, 2, 384, 64), (2, 2, 100, 80), (1, 3, 77, 96), (2, 2, 130, 128)])
 def test_recompute_dq_path_matches_oracle(dev, dt, shape):
     """With the dS workspace bound set to 0 the dQ pass recomputes S, P and
     dP from q, k, v, dO and the row statistics (the path taken above 4 GiB of
-    dS): forward and backward against the oracle at the same bar."""
+    dS), or above D = 64 the scores are materialised from the statistics that,
+    in float32, the paired-range forward left: forward and backward against
+    the oracle at the same bar."""
     D, K = _dev()
     rng = np.random.default_rng(sum(shape) + 7)
     q, k, v, g = (rng.standard_normal(shape).astype(dt) for _ in range(4))
@@ -269,8 +271,9 @@ def test_wide_heads_without_memory_for_the_ds_workspace(dev):
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 @pytest.mark.parametrize("shape", [(2, 2, 64, 128), (1, 3, 100, 80), (2, 1, 33, 256)])
 def test_head_dimensions_beyond_64(dev, dt, shape):
-    """D > 64 (e.g. dtrain's --dim 256 --heads 2): scores materialised per batch
-    element and the products as batched GEMMs; against the oracle."""
+    """D > 64 (e.g. dtrain's --dim 256 --heads 2): float64, and float32 above D =
+    128, with scores materialised per batch element and the products as batched
+    GEMMs, float32 up to D = 128 on the paired-range kernels; against the oracle."""
     D, K = _dev()
     rng = np.random.default_rng(sum(shape) + 1)
     q, k, v, g = (rng.standard_normal(shape).astype(dt) for _ in range(4))
@@ -317,11 +320,14 @@ def test_rowsum_formed_by_the_projection_gradient(dev, B, T, H, N):
 
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
-@pytest.mark.parametrize("shape", [(2, 3, 256, 64), (1, 2, 128, 32)])
+@pytest.mark.parametrize("shape", [(2, 3, 256, 64), (1, 2, 128, 32), (2, 3, 100, 64), (1, 2, 77, 48), (2, 3, 77, 80),
+                                   (1, 2, 130, 128)])
 def test_results_written_through_unaligned_views(dev, dt, shape):
     """O, dQ, dK and dV written into views one element past a 16-byte
     boundary take the element-wise stores; aligned outputs take 16-byte
-    stores. Both must give the same bits, and the values the oracle's."""
+    stores. Both must give the same bits, and the values the oracle's. dO read
+    from such a view takes the backward's general kernels (materialised scores
+    above D = 64) with the statistics of the aligned forward."""
     D, K = _dev()
     rng = np.random.default_rng(sum(shape))
     hq, hk, hv, hg = (rng.standard_normal(shape).astype(dt) for _ in range(4))
@@ -344,6 +350,10 @@ def test_results_written_through_unaligned_views(dev, dt, shape):
     ref = ops.attention_bwd(hg, hq, hk, hv, p, scale)
     assert rel_err(o2.numpy(), o_ref) <= TOL[dt]
     for a, r in zip(grads2, ref):
+        assert rel_err(a.numpy(), r) <= TOL[dt]
+    g2 = shifted()
+    g2.assign(hg)
+    for a, r in zip(K.attn_bwd(q, k, v, o, g2, rmax, rsum), ref):
         assert rel_err(a.numpy(), r) <= TOL[dt]
 
 

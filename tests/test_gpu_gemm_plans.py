@@ -1,10 +1,11 @@
 """The GEMM kernels behind the dispatch's size rules: the small-product kernel (k
 split over a block's waves), the 64 x 64 tile and the 4-byte loads of operands
 that are not 16-byte granular, at tile edges, remainders and both ends of their
-ranges, in every layout. The reference is a float64 product. The bounds are the
-worst case of a sum of K products, K u |A||B| (u the unit roundoff, eps = 2 u:
-the other half covers the float64 reference's own sum), which a lost or doubled
-term exceeds by orders of magnitude."""
+ranges, in every layout, against a float64 product twice: operands of small whole
+numbers, where every order of the sums is exact and the results must be equal (a
+lost or doubled term is at least 1), and normal ones under the worst case of a
+sum of K products, K u |A||B| (u the unit roundoff, eps = 2 u: the other half
+covers the float64 reference's own sum)."""
 import numpy as np
 import pytest
 
@@ -15,10 +16,18 @@ pytestmark = pytest.mark.gpu
 LAYOUTS = [(True, False), (True, True), (False, False), (False, True)]
 
 
-def _operands(dt, M, N, K, akc, bkc, seed):
+def _draw(rng, shape, dt, whole):
+    """Normal numbers, or whole ones of -8 to 8 without 0 (sums of up to 2^18
+    products, and of as many terms, are exact in either type)."""
+    if whole:
+        return (rng.integers(1, 9, shape) * rng.choice([-1, 1], shape)).astype(dt)
+    return rng.standard_normal(shape).astype(dt)
+
+
+def _operands(dt, M, N, K, akc, bkc, seed, whole=False):
     rng = np.random.default_rng(seed)
-    A = rng.standard_normal((M, K) if akc else (K, M)).astype(dt)
-    B = rng.standard_normal((N, K) if bkc else (K, N)).astype(dt)
+    A = _draw(rng, (M, K) if akc else (K, M), dt, whole)
+    B = _draw(rng, (N, K) if bkc else (K, N), dt, whole)
     a = (A if akc else A.T).astype(np.float64)
     b = (B.T if bkc else B).astype(a.dtype)
     return A, B, a, b
@@ -33,11 +42,15 @@ def _operands(dt, M, N, K, akc, bkc, seed):
 ])
 def test_gemm_plans_against_reference(dev, dt, akc, bkc, M, N, K):
     from dtmi import device as D, kernels as K_
-    A, B, a, b = _operands(dt, M, N, K, akc, bkc, M * 7 + N * 3 + K)
-    bias = np.random.default_rng(1).standard_normal(N).astype(dt)
-    got = K_.gemm(D.from_numpy(A), D.from_numpy(B), a_kcontig=akc, b_kcontig=bkc, bias=D.from_numpy(bias)).numpy()
-    bound = np.finfo(dt).eps * (K * (np.abs(a) @ np.abs(b)) + np.abs(bias))
-    assert np.all(np.abs(got - (a @ b + bias)) <= bound)
+    for whole in (True, False):
+        A, B, a, b = _operands(dt, M, N, K, akc, bkc, M * 7 + N * 3 + K, whole)
+        bias = _draw(np.random.default_rng(1), N, dt, whole)
+        got = K_.gemm(D.from_numpy(A), D.from_numpy(B), a_kcontig=akc, b_kcontig=bkc, bias=D.from_numpy(bias)).numpy()
+        if whole:
+            assert np.array_equal(got, a @ b + bias)
+        else:
+            bound = np.finfo(dt).eps * (K * (np.abs(a) @ np.abs(b)) + np.abs(bias))
+            assert np.all(np.abs(got - (a @ b + bias)) <= bound)
 
 
 @pytest.mark.parametrize("akc,bkc", LAYOUTS)
@@ -59,6 +72,12 @@ def test_linear_backward_column_sums_and_epilogues(dev, dt, M, K, N):
     """dW, db and dX, and the fused forward epilogues, through the small plans."""
     from dtmi import device as D, kernels as K_
     rng = np.random.default_rng(M + N)
+    x, w, g, b, r = (_draw(rng, s, dt, True) for s in ((M, K), (K, N), (M, N), (N,), (M, N)))
+    dx, dw, db = K_.linear_bwd(D.from_numpy(x), D.from_numpy(w), D.from_numpy(g))
+    assert np.array_equal(dx.numpy(), g @ w.T) and np.array_equal(dw.numpy(), x.T @ g)
+    assert np.array_equal(db.numpy(), g.sum(axis=0))
+    y, _ = K_.linear_fwd_fused(D.from_numpy(x), D.from_numpy(w), D.from_numpy(b), residual=D.from_numpy(r))
+    assert np.array_equal(y.numpy(), x @ w + b + r)
     x, w, g = (rng.standard_normal(s).astype(dt) for s in ((M, K), (K, N), (M, N)))
     b, r = rng.standard_normal(N).astype(dt), rng.standard_normal((M, N)).astype(dt)
     X, W, G = (v.astype(np.float64) for v in (x, w, g))
@@ -105,6 +124,23 @@ def test_leading_dimensions_of_2_24_bytes(dev, dt, akc, bkc, pad_a, pad_b):
         _lib.call("dtmi_gemm", _lib.dtype_code(dt), int(akc), int(bkc), M, N, K, da.ptr, ld + pad_a, 0, db.ptr,
                   ld + pad_b, 0, C.ptr, N, 0, 1, dbias.ptr, 0, splits)
         assert np.array_equal(C.numpy(), ref)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+def test_register_staged_kernel_matches_the_direct_to_lds_kernel_bitwise(dev, dt, akc, bkc):
+    """The same operands with rows 2^24 bytes apart (register-staged, as vectors)
+    and contiguous (direct to LDS): both feed the MFMAs the same k order, so the
+    products agree to the bit (one split, ragged M and N, a partial last k-tile)."""
+    from dtmi import _lib, device as D, kernels as K_
+    M, N, K = 132, 68, 200
+    A, B, _, _ = _operands(dt, M, N, K, akc, bkc, 5)
+    ld = (1 << 24) // np.dtype(dt).itemsize
+    da, db, C = _strided(A, ld), _strided(B, ld), D.empty((M, N), dt)
+    _lib.call("dtmi_gemm", _lib.dtype_code(dt), int(akc), int(bkc), M, N, K, da.ptr, ld, 0, db.ptr, ld, 0, C.ptr, N, 0,
+              1, None, 0, 1)
+    ref = K_.gemm(D.from_numpy(A), D.from_numpy(B), a_kcontig=akc, b_kcontig=bkc, splits=1)
+    assert bits_equal(C.numpy(), ref.numpy())
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])

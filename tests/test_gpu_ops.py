@@ -332,11 +332,11 @@ def test_gemm_split_k_with_partial_last_tile(dev, dt, akc, bkc):
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 @pytest.mark.parametrize("akc,bkc", [(True, False), (True, True), (False, False), (False, True)])
-def test_gemm_direct_lds_kernel_matches_register_staged_kernel_bitwise(dev, dt, akc, bkc):
-    """16-byte aligned operands take the direct-to-LDS kernel; the same values
-    one element off alignment take the register-staged kernel. Both feed the
-    MFMAs the same k order, so the products agree to the bit (128 x 128
-    block tiles, one split, ragged M and N, a partial last k-tile)."""
+def test_gemm_16_byte_and_4_byte_loads_agree_bitwise(dev, dt, akc, bkc):
+    """16-byte aligned operands go into LDS 16 bytes per lane; the same values one
+    element off alignment 4 bytes per lane, into the same layout. The products
+    agree to the bit (128 x 128 block tiles, one split, ragged M and N, a
+    partial last k-tile)."""
     D, K_ = _dev()
     rng = np.random.default_rng(41)
     M, N, K = 300, 260, 1000
@@ -349,19 +349,18 @@ def test_gemm_direct_lds_kernel_matches_register_staged_kernel_bitwise(dev, dt, 
     a_off.assign(a)
     assert a_off.ptr % 16 != 0
     aligned_ = K_.gemm(D.from_numpy(a), db, a_kcontig=akc, b_kcontig=bkc, bias=bias, splits=1).numpy()
-    staged = K_.gemm(a_off, db, a_kcontig=akc, b_kcontig=bkc, bias=bias, splits=1).numpy()
+    shifted = K_.gemm(a_off, db, a_kcontig=akc, b_kcontig=bkc, bias=bias, splits=1).numpy()
     ref = _gemm_ref(a.astype(np.float64), b.astype(np.float64), akc, bkc) + bias.numpy()
     assert rel_err(aligned_, ref) <= TOL[dt]
-    assert bits_equal(aligned_, staged)
+    assert bits_equal(aligned_, shifted)
 
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 @pytest.mark.parametrize("akc,bkc", [(True, False), (False, True)])
-def test_batched_gemm_direct_lds_kernel_matches_register_staged_kernel_bitwise(dev, dt, akc, bkc):
+def test_batched_gemm_16_byte_and_4_byte_loads_agree_bitwise(dev, dt, akc, bkc):
     """Batched products (batch strides of whole matrices, as the attention's
-    wide path uses them): the direct-to-LDS kernel on aligned operands and the
-    register-staged kernel on the same values off alignment give the same
-    bits, split into K ranges or not."""
+    wide path uses them): aligned operands and the same values off alignment
+    give the same bits, split into K ranges or not."""
     D, K_ = _dev()
     rng = np.random.default_rng(43)
     Bt, M, N, K = 3, 136, 200, 520
@@ -374,9 +373,9 @@ def test_batched_gemm_direct_lds_kernel_matches_register_staged_kernel_bitwise(d
     ref = _gemm_ref(a.astype(np.float64), b.astype(np.float64), akc, bkc)
     for splits in (1, 2):
         aligned_ = K_.gemm(D.from_numpy(a), db, a_kcontig=akc, b_kcontig=bkc, splits=splits).numpy()
-        staged = K_.gemm(a_off, db, a_kcontig=akc, b_kcontig=bkc, splits=splits).numpy()
+        shifted = K_.gemm(a_off, db, a_kcontig=akc, b_kcontig=bkc, splits=splits).numpy()
         assert rel_err(aligned_, ref) <= TOL[dt]
-        assert bits_equal(aligned_, staged)
+        assert bits_equal(aligned_, shifted)
 
 
 @pytest.mark.parametrize("akc,bkc", [(True, False), (True, True), (False, False), (False, True)])
