@@ -25,8 +25,7 @@
 // registers) and writing dS = P * (dP - rowsum(dO * O)) to a [B, H, T, T]
 // workspace; kernel B owns queries and accumulates dQ = dS K from it (when
 // the workspace would exceed its bound, kernel B recomputes dS instead).
-// Float32 with D of 36 to 128 works on 16 x 16 tiles with
-// paired ranges: key tile j and its mirror nt - 1 - j (nt + 1 tile pairs
+// Float32 with D of 36 to 128 works on 16 x 16 tiles with paired ranges: key tile j and its mirror nt - 1 - j (nt + 1 tile pairs
 // between them) split over two waves in the key pass, query tile i and its
 // mirror over a pair of waves in the dQ pass, so every wave carries the same
 // work whatever the sequence length, and dS lives in causal tiles only.
@@ -93,7 +92,7 @@ struct AttnArgs {
   void *out, *dq, *dk, *dv;
   void *rowmax, *rowsum;  // [B, H, T]
   const void* drow;       // [B, H, T] rowsum(dO * O)
-  void* ds;               // [B, H, T, T] dS written by the key-block pass for the dQ pass (or NULL)
+  void* ds;  // dS written by the key pass for the dQ pass: [B, H, T, T], or its causal 16 x 16 tiles (or NULL)
   Strides3 sq, sk, sv, so, sdo, sdq, sdk, sdv;
   int64_t B, H, T, D;
   double scale;
@@ -979,12 +978,9 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_ds_kernel(AttnArgs a) {
   store_result<T, DP, QB>(lds, dq, (T)a.scale, DQ, a.sdq.t, q0, Tn, D, wave, g, c, a.ovec != 0 && D == DP);
 }
 
-// dQ from the dS workspace, one query tile per block (float32): the block's
-// four waves take the key tiles up to the query tile in turn (wave w: tiles
-// w, w + 4, ...), each staging its key tile's rows in its own LDS region and
-// prefetching the next tile's K rows and dS entries into registers; the four
-// partial dQ are added in wave order at the end. Aligned path only (D = DP =
-// 64, T a multiple of 32, 16-byte access).
+// dQ without a dS workspace (dS above its bound): a block owns 4*MT queries (MT
+// per wave) and walks the key tiles they see, double-buffered, recomputing S, P
+// and dP per tile; dQ^T += K^T dS^T from registers.
 template <typename T, int DP, bool FAST>
 __global__ void __launch_bounds__(256, 2) attn_bwd_q_kernel(AttnArgs a) {
   using M = AM<T>;
@@ -1073,15 +1069,6 @@ __global__ void __launch_bounds__(256, 2) attn_bwd_q_kernel(AttnArgs a) {
   store_result<T, DP, QB>(lds, dq, (T)a.scale, DQ, a.sdq.t, q0, Tn, D, wave, g, c, a.ovec != 0 && D == DP);
 }
 
-// ------------------------------------------- head dimensions beyond 64
-// Where no other form applies (float64, float32 above D = 128, unaligned rows
-// or a dS above its bound) the scores of one batch element are materialised, [H, T, T] in
-// a pooled workspace, and the products run as batched GEMMs (dtmi_gemm):
-// S = Q K^T, P = softmax(S * scale + mask), O = P V; backward P recomputed
-// from S and the saved row statistics, dV = P^T dO, dP = dO V^T,
-// dS = P * (dP - rowsum(dP * P)) * scale, dQ = dS K, dK = dS^T Q -- dtrain's
-// products (autograd.py:226-246), one batch element at a time. One block per
-// row for the row passes, fixed reduction order.
 // ----------------------------- backward on 16 x 16 tiles over paired ranges
 // MFMA 16 x 16 x 4 (float32): lane (g, c), g = lane / 16, supplies column c
 // (B operand) or row c (A operand) at k-slot g, and holds column c, rows
@@ -1600,6 +1587,16 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_qp_kernel(AttnArgs a) {
   }
 }
 
+// ------------------------------------------- head dimensions beyond 64
+// Where no other form applies (float64, float32 above D = 128, unaligned rows,
+// or a dS above its bound or beyond the memory) the scores of one batch element
+// are materialised, [H, T, T] in a pooled workspace (two in the backward), and the
+// products run as batched GEMMs (dtmi_gemm):
+// S = Q K^T, P = softmax(S * scale + mask), O = P V; backward P recomputed
+// from S and the saved row statistics, dV = P^T dO, dP = dO V^T,
+// dS = P * (dP - rowsum(dP * P)) * scale, dQ = dS K, dK = dS^T Q -- dtrain's
+// products (autograd.py:226-246), one batch element at a time. One block per
+// row for the row passes, fixed reduction order.
 template <typename T>
 __device__ __forceinline__ T block_reduce_256(T x, T* red, bool is_max) {
 #pragma unroll
@@ -2068,7 +2065,7 @@ static int paired_form(const AttnArgs& a, bool backward) {
   const Strides3* st[] = {&a.sq, &a.sk, &a.sv, &a.sdo};
   for (int i = 0; i < (backward ? 4 : 3); ++i)
     if (st[i]->t < a.D || st[i]->t >= ((int64_t)1 << 29) / (a.T + 64)) return 0;
-  return a.T < (1 << 15) ? 2 : 0;  // dS of one (batch, head) below 2^31 bytes too
+  return a.T < (1 << 15) ? 2 : 0;  // dS of one (batch, head) below 2^32 bytes, the buffers' 32-bit offsets
 }
 
 template <int DP, int W, bool RAG>

@@ -277,8 +277,8 @@ __global__ void __launch_bounds__(256) reduce_group_kernel(T* __restrict__ out, 
 
 template <typename T>
 static int reduce_group(T* out, const T* x, const ReduceDesc& d, int64_t nout, int64_t nred, int64_t rs) {
-  // A part keeps at least 4096 terms (16 per thread of its block); parts are
-  // added until the blocks fill the chip.
+  // Parts of at most 4096 terms (16 per thread of a block), of more where the
+  // outputs' blocks then fill the chip.
   int64_t nparts = 1;
   if (nred >= 8192 && nout < 1024) {
     nparts = cdiv(nred, 4096);

@@ -356,9 +356,12 @@ static void pick_tile(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cu
 // traffic (about 6 TB/s from the last-level cache); where the next pass takes the
 // partials (`fused`: as LayerNorm or the row dots do), only the
 // partials beyond the output itself. Measured, 128 -> chosen:
-// [512, 512] x [512, 128] 23.9 -> 6.0 us (small-product), [1000, 256] x [256, 768]
+// [512, 384] x [384, 384] 29 -> 7 us (small-product), [1000, 256] x [256, 768]
 // float64 44.6 -> 14 us (small-product), [1500, 384] x [384, 1000] 34 -> 18 us (64),
-// [2495, 768] x [768, 768] 41 -> 29.5 us (64), [1001, 515] x [515, 1030] 36 -> 24 us.
+// [2495, 768] x [768, 768] 41 -> 33 us (64), [1001, 515] x [515, 1030] 36 -> 24 us.
+// It does not know the epilogue, nor how long one wave's chain is: over 1473 other
+// calls the geometric mean of chosen / 128 is 0.57, and the worst [2495, 1536] x
+// [1536, 384] with a LayerNorm after it, 44 -> 48 us (one 64 x 64 block per CU).
 static double tile_cost(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cus, int bm, int bn, int splits,
                         size_t es, bool fused) {
   const double k = (double)cdiv(cdiv(K, splits), 64 / (int64_t)es) * (64.0 / (double)es);
@@ -454,11 +457,15 @@ static int gemm_impl(int akc, int bkc, int64_t M, int64_t N, int64_t K, const vo
     const bool fused = tmn * batch >= cus;
     double best = 0.93 * tile_cost(M, N, K, batch, cus, bm, bn, splits, sizeof(T), fused);
     const int64_t t32 = cdiv(M, 32) * cdiv(N, 32) * batch;
-    // Float32 products with a dimension of at most 256 (every product of a small
-    // model) keep the 128-wide plan's split of k, and so its bits, whichever kernel
-    // runs: an optimizer's first steps divide gradients by their own size, which
-    // turns another rounding into another trajectory (the second step's gradients
-    // of a 4-layer model of width 128 differed by 3e-6). Others take the fastest.
+    // Float32 products with a dimension of at most 256 keep the 128-wide plan's
+    // split of k, and so the bits they had with it, whichever kernel runs. Another
+    // order of the sum is no worse a rounding (all other sizes take the fastest);
+    // what is kept is the trajectory of a small model's training run (dtrain's --dim
+    // 128 and 256): an optimizer's first steps divide gradients by their own size,
+    // and the second step's gradients of a 4-layer model of width 128 differed by
+    // 3e-6. The price, also for products that train nothing: [512, 512] x [512, 128]
+    // runs as 2 waves of 256 k, 9.9 us (6.0 split over 16, 23.7 on 128-wide tiles),
+    // [200, 384] x [384, 384] as one chain, 12 us (29; [512, 384] x [384, 384] 7).
     const bool keep = std::is_same<T, float>::value && (M <= 256 || N <= 256 || K <= 256);
     int64_t dk = kps;
     if (keep) {

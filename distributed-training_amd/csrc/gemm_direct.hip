@@ -6,11 +6,11 @@
 // on 256 CUs, and each of their waves runs K / 2 MFMAs of 64 cycles per 32 x 32
 // piece one after the other. Here a block owns one 32 x 32 tile, its nw waves
 // take consecutive ranges of k, and their partial tiles are added through LDS in
-// wave order: the four tiles become 64 blocks of up to 16 waves, with no second
-// launch to sum partials. The waves share no
-// operand data (each has its own k), so nothing is staged in LDS and there is no
-// barrier before the sum; each wave keeps one batch of k in flight in registers
-// while it multiplies the one before.
+// wave order: the four tiles become 64 blocks, of up to 16 waves where the order
+// of the sum is free (the dispatch says where), with no second launch to sum
+// partials. The waves share no operand data (each has its own k), so nothing is
+// staged in LDS and there is no barrier before the sum; each wave keeps one batch
+// of k in flight in registers while it multiplies the one before.
 //
 // Loads: a k-contiguous operand gives a lane its VEC k-values of a row as one
 // 16-byte vector, an m/n-contiguous one a k-row's 32 (16) neighbours as 4-byte
