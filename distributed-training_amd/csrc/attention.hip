@@ -1355,7 +1355,9 @@ __global__ void __launch_bounds__(64 * W, DP == 64 && W == 2 ? 3 : 2) attn_bwd_k
           dp += dp1;
         }
         auto probs = [&](auto maskc) {
-          constexpr bool MASK = decltype(maskc)::value;  // the diagonal tile
+          // the diagonal tile; RAG: and one with queries past T, whose zeros give no
+          // number against an infinite key or value
+          constexpr bool MASK = decltype(maskc)::value;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int r = M::row(i, g);
@@ -1363,12 +1365,14 @@ __global__ void __launch_bounds__(64 * W, DP == 64 && W == 2 ? 3 : 2) attn_bwd_k
             // rounded as there, times 1 / sum: the rounding of max + log2(sum),
             // a larger number, would be the probabilities' largest error
             T pr = RAG ? ex2(s[i] * sl2 - ST[r]) * ST[2 * MT + r] : ex2(__builtin_fmaf(s[i], sl2, -ST[r]));
-            if constexpr (MASK) pr = c > r ? T(0) : pr;  // key above the query: masked
+            const bool off = MASK && (RAG ? k0 + c > qs + r || qs + r >= Tn : c > r);  // key above the query
+            if constexpr (MASK) pr = off ? T(0) : pr;
             s[i] = pr;
             dp[i] = pr * (dp[i] - ST[MT + r]);
+            if constexpr (MASK && RAG) dp[i] = off ? T(0) : dp[i];
           }
         };
-        if (qt == j)
+        if (qt == j || (RAG && qs + MT > Tn))
           probs(std::true_type());
         else
           probs(std::false_type());

@@ -430,3 +430,27 @@ def test_scores_of_minus_infinity(dev, T, D_):
         for d in range(4):
             assert rel_err(got.numpy()[..., d], ref[..., d]) <= tol
         assert rel_err(got.numpy()[..., 4:], ref[..., 4:]) <= tol
+
+
+@pytest.mark.parametrize("T,D_", [(100, 36), (100, 64), (96, 64), (100, 80), (130, 128)])
+def test_keys_masked_by_an_infinite_feature(dev, T, D_):
+    """A mask carried by a feature: 1 in every query, -inf in the masked keys and
+    0 in the others. The masked keys' dK and dV are 0 and everything else is as
+    without them (dQ's own entry of that feature is 0 * inf), also where the
+    last query tile has rows past T, whose zeros times -inf are no numbers."""
+    D, K = _dev()
+    rng = np.random.default_rng(T + D_)
+    q, k, v, g = (rng.standard_normal((1, 2, T, D_)).astype(np.float32) for _ in range(4))
+    off = [3, 16, 17, 40, T - 1]
+    q[..., 0], k[..., 0] = 1, 0
+    k[:, :, off, 0] = -np.inf
+    o_ref, p, scale = ops.attention_fwd(q, k, v)
+    gq, gk, gv = ops.attention_bwd(g, q, k, v, p, scale)
+    dq_, dk_, dv_ = D.from_numpy(q), D.from_numpy(k), D.from_numpy(v)
+    o, rmax, rsum = K.attn_fwd(dq_, dk_, dv_)
+    tol = TOL[np.float32]
+    assert rel_err(o.numpy(), o_ref) <= tol
+    dq, dk, dv = (x.numpy() for x in K.attn_bwd(dq_, dk_, dv_, o, D.from_numpy(g), rmax, rsum))
+    assert rel_err(dq[..., 1:], gq[..., 1:]) <= tol
+    assert rel_err(dk, gk) <= tol and rel_err(dv, gv) <= tol
+    assert np.all(dk[:, :, off] == 0) and np.all(dv[:, :, off] == 0)
