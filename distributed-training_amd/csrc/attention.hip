@@ -97,6 +97,7 @@ struct AttnArgs {
   int64_t B, H, T, D;
   double scale;
   int vec;   // 16-byte global access allowed for every operand
+  int vec_qkv;  // for q, k and v (vec is that and dO's, in the backward)
   int head_group;  // (batch, head)s per group of the ragged forward's block order (D up to 64)
   int ovec;  // the results (out, or dq, dk and dv) too, with D a multiple of the vector
 };
@@ -1615,8 +1616,8 @@ __device__ __forceinline__ T block_reduce_256(T x, T* red, bool is_max) {
 }
 
 // Rows t of one batch element's S [H, T, T] (row r = h * T + t): P in place,
-// row statistics to rowmax / rowsum at (b * H + h) * T + t (rowmax in base-2
-// units, as the flash kernels keep it).
+// row statistics to rowmax / rowsum (if not NULL) at (b * H + h) * T + t (rowmax
+// in base-2 units, as the flash kernels keep it).
 template <typename T>
 __global__ void __launch_bounds__(256) attn_rows_softmax_kernel(T* __restrict__ S, T* __restrict__ rowmax,
                                                                  T* __restrict__ rowsum, int64_t Tn, int64_t row0,
@@ -1638,7 +1639,7 @@ __global__ void __launch_bounds__(256) attn_rows_softmax_kernel(T* __restrict__ 
   l = block_reduce_256(l, red, false);
   const T linv = T(1) / l;
   for (int64_t j = threadIdx.x; j <= t; j += 256) sr[j] = sr[j] * linv;
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && rowmax) {
     rowmax[row0 + r] = m * (T)1.4426950408889634;
     rowsum[row0 + r] = l;
   }
@@ -1733,8 +1734,11 @@ static int attn_fwd_wide(AttnArgs& a) {
   return DTMI_OK;
 }
 
+// own_stats: P from this product's own scores, where the forward's statistics are
+// of another kernel's (rounded otherwise, by up to the scores' own error: with
+// scores of 40 a row of P would not sum to 1 by 3e-6).
 template <typename T>
-static int attn_bwd_wide(AttnArgs& a) {
+static int attn_bwd_wide(AttnArgs& a, bool own_stats = false) {
   const int dt = sizeof(T) == 4 ? DTMI_F32 : DTMI_F64;
   const int64_t B = a.B, H = a.H, Tn = a.T, D = a.D;
   void* P = nullptr;
@@ -1759,8 +1763,11 @@ static int attn_bwd_wide(AttnArgs& a) {
     if (rc) break;
     {
       TimedLaunch tl(DTMI_FAM_ATTN_BWD, 0.0);
-      attn_rows_prob_kernel<T><<<(unsigned)(H * Tn), 256, 0, stream()>>>((T*)P, (const T*)a.rowmax,
-                                                                          (const T*)a.rowsum, Tn, b * H * Tn, a.scale);
+      if (own_stats)
+        attn_rows_softmax_kernel<T><<<(unsigned)(H * Tn), 256, 0, stream()>>>((T*)P, nullptr, nullptr, Tn, 0, a.scale);
+      else
+        attn_rows_prob_kernel<T><<<(unsigned)(H * Tn), 256, 0, stream()>>>(
+            (T*)P, (const T*)a.rowmax, (const T*)a.rowsum, Tn, b * H * Tn, a.scale);
     }
     // dV = P^T dO: A(m = key, k = query) = P[query][key]
     rc = gemm_call(dt, 0, 0, Tn, D, Tn, P, Tn, TT, G, a.sdo.t, a.sdo.h, dV, a.sdv.t, a.sdv.h, H);
@@ -2061,14 +2068,17 @@ static int resident_blocks(F kernel, int threads) {
 // 128 166, 169 and 189); key pass 2 (up to 64: 68 us, 74 with four, at 5, 12,
 // 499) or 4 (above: 92 us, 120 with two, at 2, 8, 777, 96; and sums of a
 // quarter of the sequence keep the error of split products).
+// q, k and v alone decide, so that a backward recomputes the scores in the order
+// that its forward's statistics and output have them in.
+static bool paired_rows(const AttnArgs& a, const Strides3& s) {
+  return s.t >= a.D && s.t < ((int64_t)1 << 29) / (a.T + 64);
+}
 template <typename T>
-static int paired_form(const AttnArgs& a, bool backward) {
-  if (sizeof(T) != 4 || !a.vec) return 0;
+static int paired_form(const AttnArgs& a) {
+  if (sizeof(T) != 4 || !a.vec_qkv) return 0;
   if (a.D == 64 && a.T % 32 == 0) return 1;
   if (a.D <= 32 || a.D > 128) return 0;
-  const Strides3* st[] = {&a.sq, &a.sk, &a.sv, &a.sdo};
-  for (int i = 0; i < (backward ? 4 : 3); ++i)
-    if (st[i]->t < a.D || st[i]->t >= ((int64_t)1 << 29) / (a.T + 64)) return 0;
+  if (!paired_rows(a, a.sq) || !paired_rows(a, a.sk) || !paired_rows(a, a.sv)) return 0;
   return a.T < (1 << 15) ? 2 : 0;  // dS of one (batch, head) below 2^32 bytes, the buffers' 32-bit offsets
 }
 
@@ -2118,7 +2128,7 @@ template <typename T>
 static int attn_fwd_impl(AttnArgs& a) {
   constexpr int MT = AM<T>::MT;
   const int dp = pick_dp<T>(a.D);
-  const int form = paired_form<T>(a, false);
+  const int form = paired_form<T>(a);
   if (dp < 0 && !form) return attn_fwd_wide<T>(a);
   dim3 grid((unsigned)cdiv(a.T, 4 * MT), (unsigned)(a.B * a.H));
   // causal-exact FLOP: 2 GEMMs of 2*D*T(T+1)/2 per (b, h)
@@ -2139,34 +2149,127 @@ static int attn_fwd_impl(AttnArgs& a) {
 // the recompute path can be exercised at any size.
 static int64_t g_max_ds_bytes = (int64_t)4 << 30;
 
+// The ragged paired-range backward in parts whose dS fits a.ds: `bhs` (batch,
+// head)s at a time, whole batch elements where they fit.
+static void attn_bwd_parts(const AttnArgs& a, int64_t bhs) {
+  const int64_t nb = bhs >= a.H ? bhs / a.H : 1, nh = bhs >= a.H ? a.H : bhs;
+  for (int64_t b = 0; b < a.B; b += nb)
+    for (int64_t h = 0; h < a.H; h += nh) {
+      AttnArgs p = a;
+      p.B = a.B - b < nb ? a.B - b : nb;
+      p.H = a.H - h < nh ? a.H - h : nh;
+      auto at = [&](const void* x, const Strides3& s) { return (float*)x + b * s.b + h * s.h; };
+      p.q = at(a.q, a.sq);
+      p.k = at(a.k, a.sk);
+      p.v = at(a.v, a.sv);
+      p.dO = at(a.dO, a.sdo);
+      p.dq = at(a.dq, a.sdq);
+      p.dk = at(a.dk, a.sdk);
+      p.dv = at(a.dv, a.sdv);
+      const int64_t row0 = (b * a.H + h) * a.T;
+      p.rowmax = (float*)a.rowmax + row0;
+      p.rowsum = (float*)a.rowsum + row0;
+      p.drow = (const float*)a.drow + row0;
+      if (a.D <= 64)
+        attn_bwd_paired<64, 2, true>(p);
+      else if (a.D <= 96)
+        attn_bwd_paired<96, 4, true>(p);
+      else
+        attn_bwd_paired<128, 4, true>(p);
+    }
+}
+
 template <typename T>
 static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
   constexpr int MT = AM<T>::MT;
   const int dp = pick_dp<T>(a.D);
-  int form = paired_form<T>(a, true);
-  // dS for the dQ pass: B*H*T*T elements (the causal tiles only on the
-  // paired-range path), up to g_max_ds_bytes; beyond that the dQ pass
-  // recomputes S, P and dP itself, or (D above 64, also where the memory for dS
-  // is not to be had) the scores of one batch element are materialised.
-  a.ds = nullptr;
-  const double ds_bytes = form ? (double)a.B * a.H * (double)ds16_tiles(2 * cdiv(a.T, 32)) * 256.0 * sizeof(T)
-                               : (double)a.B * a.H * a.T * a.T * sizeof(T);
-  const bool keep_ds = ds_bytes <= (double)g_max_ds_bytes;
-  if (!keep_ds) form = 0;
-  if (dp < 0 && !form) return attn_bwd_wide<T>(a);
-  const int64_t rows = a.B * a.H * a.T;
-  void* drow = nullptr;  // rowsum(dO * O): given, or computed below
-  int rc = drow_in ? 0 : pool_alloc(&drow, (size_t)rows * sizeof(T));
-  if (rc) return rc;
-  a.drow = drow_in ? const_cast<void*>(drow_in) : drow;
-  if (keep_ds) {
-    rc = pool_alloc(&a.ds, (size_t)ds_bytes);
-    if (rc) {
-      pool_free(drow);
-      // materialised scores need two [H, T, T] arrays, whatever the batch
-      return dp < 0 && rc == DTMI_ERR_OOM ? attn_bwd_wide<T>(a) : rc;
+  const int64_t bh = a.B * a.H, rows = bh * a.T;
+  const int fwd_form = paired_form<T>(a);
+  int form = fwd_form == 1 && !a.vec ? 0 : fwd_form;
+  // what this call allocates from the pool, given back at its end
+  void* own[4] = {};
+  int nown = 0;
+  auto take = [&](void** p, size_t bytes) {
+    const int rc = pool_alloc(p, bytes);
+    if (!rc) own[nown++] = *p;
+    return rc;
+  };
+  auto done = [&](int rc) {
+    while (nown > 0) pool_free(own[--nown]);
+    return rc;
+  };
+  const Strides3 packed{a.H * a.T * a.D, a.T * a.D, a.D};
+  if (form == 2 && !(a.vec && paired_rows(a, a.sdo))) {
+    // dO off the 16-byte grid, or rows that overlap (an expanded gradient): packed
+    void* g = nullptr;
+    if (take(&g, (size_t)(rows * a.D) * sizeof(T)) == 0) {
+      const int64_t shape[4] = {a.B, a.H, a.T, a.D}, src[4] = {a.sdo.b, a.sdo.h, a.sdo.t, 1};
+      const int rc = dtmi_copy_strided(DTMI_F32, g, nullptr, a.dO, src, 4, shape);
+      if (rc) return done(rc);
+      a.dO = g;
+      a.sdo = packed;
+      a.vec = 1;
+    } else {
+      form = 0;
     }
   }
+  // dS for the dQ pass: B*H*T*T elements, or the causal tiles on the paired-range
+  // path, up to g_max_ds_bytes. Beyond that (or beyond the memory) the ragged
+  // paired-range path takes as many (batch, head)s at a time as fit; where not even
+  // one does, and on the other paths, the dQ pass recomputes S, P and dP itself, or
+  // (D above 64) the scores of one batch element are materialised.
+  a.ds = nullptr;
+  const double bh_bytes = form ? (double)ds16_tiles(2 * cdiv(a.T, 32)) * 256.0 * sizeof(T)
+                               : (double)a.T * a.T * sizeof(T);
+  int64_t part = bh;  // (batch, head)s per dS
+  if (form == 2) {
+    const double fit = (double)g_max_ds_bytes / bh_bytes;
+    part = fit < (double)bh ? (int64_t)fit : bh;
+    for (; part > 0; part /= 8) {
+      if (part > a.H) part -= part % a.H;
+      const int rc = take(&a.ds, (size_t)part * (size_t)bh_bytes);
+      if (rc == 0) break;
+      if (rc != DTMI_ERR_OOM) return done(rc);
+    }
+    if (part == 0) form = 0;
+  }
+  if (form != 2) {
+    const double ds_bytes = (double)bh * (form ? bh_bytes : (double)a.T * a.T * sizeof(T));
+    const bool keep_ds = ds_bytes <= (double)g_max_ds_bytes;
+    if (!keep_ds) form = 0;
+    if (dp < 0 && !form) return done(attn_bwd_wide<T>(a, fwd_form == 2));
+    if (fwd_form == 2) {
+      // the general kernels after a paired-range forward: with the statistics and
+      // output of their own forward (given ones if there is no memory for it)
+      void *o = nullptr, *m = nullptr;
+      if (take(&o, (size_t)(rows * a.D) * sizeof(T)) == 0 && take(&m, (size_t)(2 * rows) * sizeof(T)) == 0) {
+        TimedLaunch tl(DTMI_FAM_ATTN_FWD, 2.0 * 2.0 * bh * a.D * (double)a.T * (a.T + 1) / 2.0);
+        const AttnArgs b = a;
+        a.out = o;
+        a.so = packed;
+        a.rowmax = m;
+        a.rowsum = (T*)m + rows;
+        a.vec = a.vec_qkv;
+        a.ovec = 1;
+        dim3 grid((unsigned)cdiv(a.T, 4 * MT), (unsigned)bh);
+        DP_SWITCH(dp, attn_fwd_kernel, T, grid)
+        a.o = o;
+        a.vec = b.vec;
+        a.ovec = b.ovec;
+        drow_in = nullptr;
+      }
+    }
+    if (keep_ds) {
+      const int rc = take(&a.ds, (size_t)ds_bytes);
+      if (rc) return done(rc);
+    }
+  }
+  void* drow = nullptr;  // rowsum(dO * O): given, or computed below
+  if (!drow_in) {
+    const int rc = pool_alloc(&drow, (size_t)rows * sizeof(T));
+    if (rc) return done(rc);
+  }
+  a.drow = drow_in ? const_cast<void*>(drow_in) : drow;
   {
     // causal-exact FLOP of the 5 backward GEMMs (S recompute, dV, dP, dQ, dK)
     TimedLaunch tl(DTMI_FAM_ATTN_BWD, 5.0 * 2.0 * a.B * a.H * a.D * (double)a.T * (a.T + 1) / 2.0);
@@ -2183,12 +2286,7 @@ static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
     if (form == 1) {
       attn_bwd_paired<64, 2, false>(a);
     } else if (form == 2) {
-      if (a.D <= 64)
-        attn_bwd_paired<64, 2, true>(a);
-      else if (a.D <= 96)
-        attn_bwd_paired<96, 4, true>(a);
-      else
-        attn_bwd_paired<128, 4, true>(a);
+      attn_bwd_parts(a, part);
     } else {
       // 128-key (128-query) blocks; the dQ pass reads dS, or recomputes it
       // above the workspace bound
@@ -2206,9 +2304,8 @@ static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
   }
   hipError_t le = hipGetLastError();
   pool_free(drow);
-  if (a.ds) pool_free(a.ds);
-  if (le != hipSuccess) return fail_hip(le, "attention backward kernels", __FILE__, __LINE__);
-  return DTMI_OK;
+  if (le != hipSuccess) return done(fail_hip(le, "attention backward kernels", __FILE__, __LINE__));
+  return done(DTMI_OK);
 }
 
 static Strides3 s3(const int64_t* s) { return Strides3{s[0], s[1], s[2]}; }
@@ -2249,6 +2346,7 @@ DTMI_EXPORT int dtmi_attn_fwd(int dtype, int64_t B, int64_t H, int64_t T, int64_
            strides_vec(a.sk, vecn) && strides_vec(a.sv, vecn))
               ? 1
               : 0;
+  a.vec_qkv = a.vec;
   a.ovec = (D % vecn == 0 && aligned(o, 16) && strides_vec(a.so, vecn)) ? 1 : 0;
   if (dtype == DTMI_F32) return attn_fwd_impl<float>(a);
   return attn_fwd_impl<double>(a);
@@ -2293,11 +2391,11 @@ static int attn_bwd_entry(int dtype, int64_t B, int64_t H, int64_t T, int64_t D,
   a.D = D;
   a.scale = scale;
   const int64_t vecn = dtype == DTMI_F32 ? 4 : 2;
-  a.vec = (D % vecn == 0 && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && aligned(dO, 16) &&
-           strides_vec(a.sq, vecn) && strides_vec(a.sk, vecn) && strides_vec(a.sv, vecn) &&
-           strides_vec(a.sdo, vecn))
-              ? 1
-              : 0;
+  a.vec_qkv = (D % vecn == 0 && aligned(q, 16) && aligned(k, 16) && aligned(v, 16) && strides_vec(a.sq, vecn) &&
+               strides_vec(a.sk, vecn) && strides_vec(a.sv, vecn))
+                  ? 1
+                  : 0;
+  a.vec = (a.vec_qkv && aligned(dO, 16) && strides_vec(a.sdo, vecn)) ? 1 : 0;
   a.ovec = (D % vecn == 0 && aligned(dq, 16) && aligned(dk, 16) && aligned(dv, 16) && strides_vec(a.sdq, vecn) &&
             strides_vec(a.sdk, vecn) && strides_vec(a.sdv, vecn))
                ? 1

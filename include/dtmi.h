@@ -405,13 +405,15 @@ int dtmi_attn_bwd_rowsum(int dtype, int64_t B, int64_t H, int64_t T, int64_t D, 
                          void* dq, const int64_t* dq_strides, void* dk, const int64_t* dk_strides, void* dv,
                          const int64_t* dv_strides);
 /* The backward's dQ pass reads the dS = P * (dP - rowsum(dO * O)) that its key
- * pass wrote to a pooled [B, H, T, T] workspace (float32 with D of 36 to 128 and
- * 16-byte aligned rows: its causal half) when that takes at most `bytes`
+ * pass wrote to a pooled [B, H, T, T] workspace when that takes at most `bytes`
  * (default 4 GiB), and otherwise recomputes S, P and dP itself (the same
- * products as dtrain/autograd.py:239-246). Above D = 64 the other way is
- * materialised scores, two pooled [H, T, T] arrays; float32 takes it also where
- * the workspace cannot be allocated. Sets the bound (0: always recompute) and
- * returns the previous one in *previous (if not NULL). */
+ * products as dtrain/autograd.py:239-246) or, above D = 64, materialises the
+ * scores of one batch element in two pooled [H, T, T] arrays. float32 with D of
+ * 36 to 128 and 16-byte aligned q, k and v rows keeps the causal half only and,
+ * where that is above the bound or cannot be allocated, works on as many (batch,
+ * head)s at a time as fit (D = 64 with T a multiple of 32: recomputes). Sets the
+ * bound (0: always recompute) and returns the previous one in *previous (if not
+ * NULL). */
 int dtmi_attn_set_ds_limit(int64_t bytes, int64_t* previous);
 
 #ifdef __cplusplus

@@ -200,9 +200,8 @@ def test_attention_on_fused_qkv_layout(dev, dt):
 def test_recompute_dq_path_matches_oracle(dev, dt, shape):
     """With the dS workspace bound set to 0 the dQ pass recomputes S, P and
     dP from q, k, v, dO and the row statistics (the path taken above 4 GiB of
-    dS), or above D = 64 the scores are materialised from the statistics that,
-    in float32, the paired-range forward left: forward and backward against
-    the oracle at the same bar."""
+    dS), or above D = 64 the scores are materialised: forward and backward
+    against the oracle at the same bar."""
     D, K = _dev()
     rng = np.random.default_rng(sum(shape) + 7)
     q, k, v, g = (rng.standard_normal(shape).astype(dt) for _ in range(4))
@@ -238,13 +237,11 @@ def test_backward_without_the_ds_workspace_matches_with_it(dev):
         assert rel_err(full.numpy(), ref) <= 1e-5
 
 
-def test_wide_heads_without_memory_for_the_ds_workspace(dev):
-    """D above 64 where dS of the whole batch (576 batch elements of T 16384:
-    309 GB) cannot be allocated: the backward falls back to materialised scores,
-    two [H, T, T] arrays whatever the batch. The batch elements share their
-    inputs (stride 0), so each one's gradients are those of a batch of one by
-    the same route (bound 0), to the bit, and those of the dS route to the
-    float32 bar."""
+def test_ragged_backward_without_memory_for_the_ds_workspace(dev):
+    """dS of the whole batch (576 batch elements of T 16384: 309 GB) cannot be
+    allocated: the backward takes as many batch elements at a time as can. The
+    batch elements share their inputs (stride 0), so each one's gradients are
+    those of a batch of one, to the bit."""
     D, K = _dev()
     B, T, Dh = 576, 16384, 72
     rng = np.random.default_rng(72)
@@ -254,18 +251,75 @@ def test_wide_heads_without_memory_for_the_ds_workspace(dev):
     def batch(x):
         return D.DeviceArray(x.block, (B, 1, T, Dh), x.dtype, x.offset, (0, T * Dh, Dh, 1))
     stats = [D.from_numpy(np.ascontiguousarray(np.broadcast_to(x.numpy(), (B, 1, T)))) for x in (m1, l1)]
-    by_ds = K.attn_bwd(q1, k1, v1, o1, g1, m1, l1)
+    one = K.attn_bwd(q1, k1, v1, o1, g1, m1, l1)
     prev = K.attn_set_ds_limit(1 << 50)
     try:
         got = K.attn_bwd(*(batch(x) for x in (q1, k1, v1, o1, g1)), *stats)
-        K.attn_set_ds_limit(0)
-        one = K.attn_bwd(q1, k1, v1, o1, g1, m1, l1)
     finally:
         K.attn_set_ds_limit(prev)
-    for x, r, d in zip(got, one, by_ds):
-        for b in (0, B - 1):
+    for x, r in zip(got, one):
+        for b in (0, 100, B - 1):
             assert bits_equal(x[b].numpy(), r[0].numpy())
-        assert rel_err(r.numpy(), d.numpy()) <= TOL[np.float32]
+
+
+@pytest.mark.parametrize("shape", [(5, 3, 100, 64), (5, 3, 77, 80), (2, 3, 130, 128)])
+@pytest.mark.parametrize("heads", [1, 2, 3, 4, 7])
+def test_ragged_backward_in_parts_of_the_batch(dev, shape, heads):
+    """A dS bound of a few (batch, head)s: parts of heads of one batch element,
+    of whole batch elements, and a smaller last part, to the bit as at once."""
+    D, K = _dev()
+    B, H, T, _ = shape
+    rng = np.random.default_rng(sum(shape))
+    # q, k, v and the gradients' buffers as views of a [B, T, 3, H, D] projection
+    qkv = D.from_numpy(rng.standard_normal((B, T, 3, H, shape[3])).astype(np.float32)).transpose(2, 0, 3, 1, 4)
+    g = D.from_numpy(rng.standard_normal((B, T, H, shape[3])).astype(np.float32)).transpose(0, 2, 1, 3)
+    o, rmax, rsum = K.attn_fwd(qkv[0], qkv[1], qkv[2])
+
+    def bwd():
+        buf = D.full((B, T, 3, H, shape[3]), 7.0, np.float32)
+        d5 = buf.transpose(2, 0, 3, 1, 4)
+        K.attn_bwd(qkv[0], qkv[1], qkv[2], o, g, rmax, rsum, dq=d5[0], dk=d5[1], dv=d5[2])
+        return buf.numpy()
+    whole = bwd()
+    nt = 2 * -(-T // 32)
+    prev = K.attn_set_ds_limit(heads * nt * (nt + 1) // 2 * 1024)
+    try:
+        assert bits_equal(bwd(), whole)
+    finally:
+        K.attn_set_ds_limit(prev)
+
+
+@pytest.mark.parametrize("T,D_", [(47, 48), (63, 64), (65, 72), (100, 128)])
+@pytest.mark.parametrize("route", ["aligned", "unaligned dO", "expanded dO", "no dS"])
+def test_backward_probabilities_sum_to_one_by_every_route(dev, T, D_, route):
+    """With dO[r, d] = 1 for d = r the sum of dV's column r is the sum of row r of
+    the probabilities that the backward recomputed. At scores of up to a few
+    hundred, rounded to 1e-5, it is 1 to a float32 sum's error (T terms of at most
+    1, each off by a few units in the last place) only if the statistics are of
+    scores added in the backward's own order; so whatever route the backward
+    takes, they have to be. "expanded": dO's rows overlap in memory."""
+    D, K = _dev()
+    rng = np.random.default_rng(T)
+    q, k, v = (D.from_numpy((3 * rng.standard_normal((1, 2, T, D_))).astype(np.float32)) for _ in range(3))
+    o, rmax, rsum = K.attn_fwd(q, k, v, scale=1.0)
+    eye = np.broadcast_to(np.eye(T, D_, dtype=np.float32), (1, 2, T, D_))
+    if route == "unaligned dO":
+        g = D.empty((2 * T * D_ + 1,), np.float32)[1:].reshape(1, 2, T, D_)
+        g.assign(eye)
+    elif route == "expanded dO":  # row r starts one element before row r - 1
+        line = np.zeros(T + D_, np.float32)
+        line[T] = 1
+        buf = D.from_numpy(line)
+        g = D.DeviceArray(buf.block, (1, 2, T, D_), np.float32, 4 * T, (0, 0, -1, 1))
+    else:
+        g = D.from_numpy(np.ascontiguousarray(eye))
+    prev = K.attn_set_ds_limit(0 if route == "no dS" else 4 << 30)
+    try:
+        dv = K.attn_bwd(q, k, v, o, g, rmax, rsum, scale=1.0)[2].numpy()
+    finally:
+        K.attn_set_ds_limit(prev)
+    sums = dv.astype(np.float64).sum(axis=2)[..., :min(T, D_)]
+    assert np.max(np.abs(sums - 1)) <= 8 * np.finfo(np.float32).eps
 
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
@@ -326,8 +380,8 @@ def test_results_written_through_unaligned_views(dev, dt, shape):
     """O, dQ, dK and dV written into views one element past a 16-byte
     boundary take the element-wise stores; aligned outputs take 16-byte
     stores. Both must give the same bits, and the values the oracle's. dO read
-    from such a view takes the backward's general kernels (materialised scores
-    above D = 64) with the statistics of the aligned forward."""
+    from such a view is packed first on the ragged paired-range path (the same
+    bits) and takes the general kernels elsewhere."""
     D, K = _dev()
     rng = np.random.default_rng(sum(shape))
     hq, hk, hv, hg = (rng.standard_normal(shape).astype(dt) for _ in range(4))
@@ -353,8 +407,10 @@ def test_results_written_through_unaligned_views(dev, dt, shape):
         assert rel_err(a.numpy(), r) <= TOL[dt]
     g2 = shifted()
     g2.assign(hg)
-    for a, r in zip(K.attn_bwd(q, k, v, o, g2, rmax, rsum), ref):
+    for a, r, b in zip(K.attn_bwd(q, k, v, o, g2, rmax, rsum), ref, grads):
         assert rel_err(a.numpy(), r) <= TOL[dt]
+        if dt == np.float32 and 32 < shape[3] <= 128 and (shape[3] != 64 or shape[2] % 32):
+            assert bits_equal(a.numpy(), b.numpy())
 
 
 @pytest.mark.parametrize("D_", [36, 64, 80, 96, 100, 128])
