@@ -2128,7 +2128,8 @@ template <typename T>
 static int attn_fwd_impl(AttnArgs& a) {
   constexpr int MT = AM<T>::MT;
   const int dp = pick_dp<T>(a.D);
-  const int form = paired_form<T>(a);
+  int form = paired_form<T>(a);
+  if (dp < 0 && a.so.t < a.D) form = 0;  // rows that overlap: for the products to refuse
   if (dp < 0 && !form) return attn_fwd_wide<T>(a);
   dim3 grid((unsigned)cdiv(a.T, 4 * MT), (unsigned)(a.B * a.H));
   // causal-exact FLOP: 2 GEMMs of 2*D*T(T+1)/2 per (b, h)
@@ -2186,6 +2187,7 @@ static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
   const int64_t bh = a.B * a.H, rows = bh * a.T;
   const int fwd_form = paired_form<T>(a);
   int form = fwd_form == 1 && !a.vec ? 0 : fwd_form;
+  if (dp < 0 && (a.sdo.t < a.D || a.sdq.t < a.D || a.sdk.t < a.D || a.sdv.t < a.D)) form = 0;  // as in the forward
   // what this call allocates from the pool, given back at its end
   void* own[4] = {};
   int nown = 0;
@@ -2200,7 +2202,8 @@ static int attn_bwd_impl(AttnArgs& a, const void* drow_in) {
   };
   const Strides3 packed{a.H * a.T * a.D, a.T * a.D, a.D};
   if (form == 2 && !(a.vec && paired_rows(a, a.sdo))) {
-    // dO off the 16-byte grid, or rows that overlap (an expanded gradient): packed
+    // dO off the 16-byte grid, or (D up to 64) rows that overlap, as an expanded
+    // gradient's do: packed
     void* g = nullptr;
     if (take(&g, (size_t)(rows * a.D) * sizeof(T)) == 0) {
       const int64_t shape[4] = {a.B, a.H, a.T, a.D}, src[4] = {a.sdo.b, a.sdo.h, a.sdo.t, 1};

@@ -313,6 +313,10 @@ def test_backward_probabilities_sum_to_one_by_every_route(dev, T, D_, route):
         g = D.DeviceArray(buf.block, (1, 2, T, D_), np.float32, 4 * T, (0, 0, -1, 1))
     else:
         g = D.from_numpy(np.ascontiguousarray(eye))
+    if route == "expanded dO" and D_ > 64:  # the batched products have never taken such rows
+        with pytest.raises(Exception, match="too small"):
+            K.attn_bwd(q, k, v, o, g, rmax, rsum, scale=1.0)
+        return
     prev = K.attn_set_ds_limit(0 if route == "no dS" else 4 << 30)
     try:
         dv = K.attn_bwd(q, k, v, o, g, rmax, rsum, scale=1.0)[2].numpy()
@@ -510,3 +514,20 @@ def test_keys_masked_by_an_infinite_feature(dev, T, D_):
     assert rel_err(dq[..., 1:], gq[..., 1:]) <= tol
     assert rel_err(dk, gk) <= tol and rel_err(dv, gv) <= tol
     assert np.all(dk[:, :, off] == 0) and np.all(dv[:, :, off] == 0)
+
+
+@pytest.mark.parametrize("D_", [80, 128])
+def test_results_with_overlapping_rows_are_refused_above_64(dev, D_):
+    """Output rows less than D apart: refused above D = 64 in the forward and the
+    backward, in float32 as in float64."""
+    D, K = _dev()
+    T = 40
+    for dt in (np.float32, np.float64):
+        q, k, v, g = (D.full((1, 1, T, D_), 0.5, dt) for _ in range(4))
+        bad = D.DeviceArray(D.full((T * D_,), 0.0, dt).block, (1, 1, T, D_), dt, 0, (0, 0, D_ - 16, 1))
+        with pytest.raises(Exception, match="ldc"):
+            K.attn_fwd(q, k, v, out=bad)
+        o, rmax, rsum = K.attn_fwd(q, k, v)
+        for i in range(3):
+            with pytest.raises(Exception, match="ldc"):
+                K.attn_bwd(q, k, v, o, g, rmax, rsum, **{("dq", "dk", "dv")[i]: bad})
