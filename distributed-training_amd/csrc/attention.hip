@@ -2019,7 +2019,9 @@ __global__ void __launch_bounds__(64 * W, DP == 64 ? 1 : 2) attn_fwd_p16_kernel(
       }
       if (g == 0 && wave == 0) {
         ((float*)a.rowmax)[(int64_t)bh * Tn + q0 + c] = mtop;
-        ((float*)a.rowsum)[(int64_t)bh * Tn + q0 + c] = l == 0.f ? kNone : l * ex2(mref - mtop);
+        float sum = l * ex2(mref - mtop);  // NaN (0 * inf) without a finite score: as kNone
+        if constexpr (kNone == 0.f) sum = l == 0.f ? 0.f : sum;
+        ((float*)a.rowsum)[(int64_t)bh * Tn + q0 + c] = sum;
       }
     }
     wave_sync();  // the last tile's rows are read before the next segment's put
